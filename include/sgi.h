@@ -310,7 +310,7 @@ typedef struct sgi_triangles {
  * distance: F32, F16 or UNORM16 (the reference's GL_DEPTH_COMPONENT16);
  * diffuse: RGBA8 atlases of the same geometry, or NULL.  nearPlane:
  * SGI_REFERENCE_VPL_NEAR_PLANE in the reference.  The context keeps a list
- * workspace (about 24 B per triangle per light of a batch, batches within
+ * workspace (about 48 B per triangle per light of a batch, batches within
  * 256 MB), allocated on first use. */
 int sgi_render_vpl_cubes(sgi_ctx* ctx, const sgi_triangles* mesh, const sgi_vpl* vpls, const int32_t* updates,
                          int32_t numUpdates, const sgi_atlas_entry* entries, float nearPlane,
@@ -332,7 +332,7 @@ int sgi_render_vpl_cubes(sgi_ctx* ctx, const sgi_triangles* mesh, const sgi_vpl*
  * all of one sign.  The shader's alpha test and the dynamic meshes do not
  * apply (static, opaque triangles).  slopeFactor:
  * SGI_REFERENCE_CSM_SLOPE_FACTOR in the reference.  The context keeps a
- * workspace of 160 B per triangle, allocated on first use. */
+ * workspace of 192 B per triangle, allocated on first use. */
 int sgi_render_csm(sgi_ctx* ctx, const sgi_triangles* mesh, const sgi_csm* csm, float slopeFactor, float* depth,
                    void* stream);
 

@@ -1,0 +1,83 @@
+"""The shadow passes' tile drawing at its edges, bit for bit the oracle's brute-force restatement:
+resolutions that end within a region, a tile and a lane's 2x2 texels, one wave per tile and four
+(the calls with many tiles and with few), triangle lists shorter and longer than a wave's scan,
+double-sided meshes (view depths of both signs) and an empty list."""
+import dataclasses
+
+import numpy as np
+import pytest
+
+import oracle as orc
+from gpu_util import require_gpu
+from stratusgfx_amd import _abi
+from stratusgfx_amd import scene as sc
+from stratusgfx_amd.gi import GiPass
+
+pytestmark = pytest.mark.gpu
+
+
+def _city(boxes, lights=4):
+    s = sc.Scene(dataclasses.replace(sc.CITY_1080P, num_vpls=lights, num_city_boxes=boxes, city_half_extent=40.0))
+    pos, col = s.triangles()
+    return s, pos, col
+
+
+def _atlases(layers, res, fmt, alloc):
+    z, c = alloc((layers, 6, res, res), fmt), alloc((layers, 6, res, res), None)
+    cz, cc = _abi.CubeAtlases(), _abi.CubeAtlases()
+    for a, f, t in ((cz, fmt, z), (cc, _abi.TEXEL_RGBA8, c)):
+        a.resolution, a.format, a.layers_per_atlas, a.num_atlases = res, f, layers, 1
+        a.atlas[0] = t.ctypes.data if isinstance(t, np.ndarray) else t.data_ptr()
+    return z, c, cz, cc
+
+
+@pytest.mark.parametrize("res,lights,boxes,fmt,cull", [
+    (1, 1, 30, _abi.TEXEL_F32, _abi.CULLING_CCW), (15, 3, 30, _abi.TEXEL_UNORM16, _abi.CULLING_NONE),
+    (17, 2, 200, _abi.TEXEL_F16, _abi.CULLING_CW), (33, 2, 200, _abi.TEXEL_UNORM16, _abi.CULLING_CCW),
+    (47, 2, 200, _abi.TEXEL_F32, _abi.CULLING_NONE), (194, 40, 60, _abi.TEXEL_F16, _abi.CULLING_CCW),
+    (194, 40, 0, _abi.TEXEL_UNORM16, _abi.CULLING_CCW)])
+def test_cubes(res, lights, boxes, fmt, cull):
+    torch = require_gpu()
+    s, pos, col = _city(max(boxes, 1), lights)
+    if boxes == 0:
+        pos, col = pos[:0], col[:0]
+    vpls, _ = s.vpls()
+    ent = np.stack([np.zeros(lights, np.int32), np.arange(lights, dtype=np.int32)], 1)
+    kinds = {_abi.TEXEL_F32: torch.float32, _abi.TEXEL_F16: torch.float16, _abi.TEXEL_UNORM16: torch.int16,
+             None: torch.int32}
+    z, c, cz, cc = _atlases(lights, res, fmt, lambda sh, f: torch.full(sh, 3, dtype=kinds[f], device="cuda"))
+    d = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()  # noqa: E731
+    none = boxes == 0
+    print(f"[tiles] cubes res {res} lights {lights} triangles {pos.shape[0]} fmt {fmt} cull {cull}", flush=True)
+    GiPass(64, 64).render_vpl_cubes(None if none else d(pos), None if none else d(col.view(np.int32)), d(vpls),
+                                    d(np.arange(lights, dtype=np.int32)), d(ent), cz, cc, cull=cull)
+    torch.cuda.synchronize()
+    hk = {_abi.TEXEL_F32: np.float32, _abi.TEXEL_F16: np.float16, _abi.TEXEL_UNORM16: np.uint16, None: np.uint32}
+    hz, hc, hcz, hcc = _atlases(lights, res, fmt, lambda sh, f: np.zeros(sh, hk[f]))
+    pick = np.array(sorted({0, lights // 2, lights - 1}), np.int32)
+    orc.render_vpl_cubes(pos, col, vpls, pick, ent, _abi.REFERENCE_VPL_NEAR_PLANE, hcz, hcc, cull=cull)
+    got, colour = z.cpu().numpy(), c.cpu().numpy().view(np.uint32)
+    for u in pick:
+        assert got[u].tobytes() == hz[u].tobytes(), f"distance of light {u}"
+        assert np.array_equal(colour[u], hc[u]), f"colour of light {u}"
+
+
+@pytest.mark.parametrize("res,boxes,cull", [(1, 30, _abi.CULLING_CCW), (31, 200, _abi.CULLING_NONE),
+                                            (33, 200, _abi.CULLING_CW), (113, 200, _abi.CULLING_CCW),
+                                            (1442, 8, _abi.CULLING_CCW), (50, 0, _abi.CULLING_CCW)])
+def test_cascades(res, boxes, cull):
+    torch = require_gpu()
+    s, pos, _ = _city(max(boxes, 1))
+    if boxes == 0:
+        pos = pos[:0]
+    csm = _abi.Csm()
+    csm.resolution = res
+    for k in range(4):
+        for i in range(16):
+            csm.cascadeProjViews[k][i] = s.csm.cascadeProjViews[k][i]
+    depth = torch.full((4, res, res), -3.0, dtype=torch.float32, device="cuda")
+    print(f"[tiles] cascades res {res} triangles {pos.shape[0]} cull {cull}", flush=True)
+    GiPass(64, 64).render_csm(torch.from_numpy(pos).cuda() if boxes else None, csm, depth, cull=cull)
+    torch.cuda.synchronize()
+    want = orc.render_csm(pos, csm, slope=_abi.REFERENCE_CSM_SLOPE_FACTOR, cull=cull)
+    assert np.array_equal(depth.cpu().numpy().view(np.uint32), want.view(np.uint32))
