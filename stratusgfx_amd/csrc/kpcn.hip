@@ -174,31 +174,9 @@ __device__ __forceinline__ void softmax25(const float* lg, float* wgt) {
     for (int j = 0; j < SGI_KPCN_TAPS; ++j) wgt[j] *= inv;
 }
 
-__device__ __forceinline__ void loadLogits(const float* logits, size_t p, float* lg) {
-    const float4* src = reinterpret_cast<const float4*>(logits + p * kC);
-#pragma unroll
-    for (int j = 0; j < 7; ++j) {
-        const float4 v = src[j];
-        lg[4 * j] = v.x;
-        lg[4 * j + 1] = v.y;
-        lg[4 * j + 2] = v.z;
-        lg[4 * j + 3] = v.w;
-    }
-}
-
 // One filter tap: o + v w per channel, one rounding each (FMA).
 __device__ __forceinline__ f3 fmaTap(f3 v, float w, f3 o) {
     return f3{__builtin_fmaf(v.x, w, o.x), __builtin_fmaf(v.y, w, o.y), __builtin_fmaf(v.z, w, o.z)};
-}
-
-__device__ __forceinline__ f3 filtered(const float* radiance, int W, int H, int x, int y, const float* wgt) {
-    f3 o = splat(0.0f);
-#pragma unroll
-    for (int j = 0; j < SGI_KPCN_TAPS; ++j) {
-        const int xx = min(max(x + j % 5 - 2, 0), W - 1), yy = min(max(y + j / 5 - 2, 0), H - 1);
-        o = fmaTap(ld3(radiance + 3 * ((size_t)yy * W + xx)), wgt[j], o);
-    }
-    return o;
 }
 
 // One axis of 2x bilinear upsampling: fine pixel x samples the coarser grid
@@ -214,62 +192,8 @@ __device__ __forceinline__ void bilinearAxis(int x, int n, int& i0, int& i1, flo
     i1 = min(max(a + 1, 0), n - 1);
 }
 
-// up(coarse) at fine pixel (x, y); T.coarse(X, Y) reads the coarser level
-// ((h, w) its size) at in-range coordinates.
-template <class T>
-__device__ __forceinline__ f3 upBilinearT(const T& src, int h, int w, int x, int y) {
-    int y0, y1, x0, x1;
-    float wy0, wy1, wx0, wx1;
-    bilinearAxis(y, h, y0, y1, wy0, wy1);
-    bilinearAxis(x, w, x0, x1, wx0, wx1);
-    const f3 top = src.coarse(x0, y0) * wx0 + src.coarse(x1, y0) * wx1;
-    const f3 bot = src.coarse(x0, y1) * wx0 + src.coarse(x1, y1) * wx1;
-    return top * wy0 + bot * wy1;
-}
-
 __device__ __forceinline__ float sigmoidf(float x) {
     return 1.0f / (1.0f + __builtin_amdgcn_exp2f(gmin(-x * kLog2e, 126.0f)));
-}
-
-// One level of the reconstruction at pixel (x, y): the 5x5 softmax filter of
-// this level's radiance, blended with the upsampled coarser output when given.
-// T.radiance(xx, yy) reads the level's radiance at in-image coordinates.
-template <class T>
-__device__ __forceinline__ f3 composePixelT(const float* lg, const T& src, bool hasCoarse, int W, int H, int x,
-                                            int y) {
-    float wgt[SGI_KPCN_TAPS];
-    softmax25(lg, wgt);
-    f3 o = splat(0.0f);
-#pragma unroll
-    for (int j = 0; j < SGI_KPCN_TAPS; ++j) {
-        const int xx = min(max(x + j % 5 - 2, 0), W - 1), yy = min(max(y + j / 5 - 2, 0), H - 1);
-        o = fmaTap(src.radiance(xx, yy), wgt[j], o);
-    }
-    if (hasCoarse) {
-        const float b = sigmoidf(lg[SGI_KPCN_BLEND_CHANNEL]);
-        o = o + (upBilinearT(src, (H + 1) / 2, (W + 1) / 2, x, y) - o) * b;
-    }
-    return o;
-}
-
-// The same taps read from global memory.
-struct GlobalTaps {
-    const float* rad;
-    const float* co;
-    int W, cw;
-    __device__ __forceinline__ f3 radiance(int xx, int yy) const { return ld3(rad + 3 * ((size_t)yy * W + xx)); }
-    __device__ __forceinline__ f3 coarse(int X, int Y) const { return ld3(co + 3 * ((size_t)Y * cw + X)); }
-};
-
-__device__ __forceinline__ f3 upBilinear(const float* __restrict__ coarse, int h, int w, int x, int y) {
-    const GlobalTaps t{nullptr, coarse, 0, w};
-    return upBilinearT(t, h, w, x, y);
-}
-
-__device__ __forceinline__ f3 composePixel(const float* lg, const float* __restrict__ radiance,
-                                           const float* __restrict__ coarse, int W, int H, int x, int y) {
-    const GlobalTaps t{radiance, coarse, W, (W + 1) / 2};
-    return composePixelT(lg, t, coarse != nullptr, W, H, x, y);
 }
 
 // Where the convolution's input comes from (staged into the LDS halo):
@@ -286,7 +210,7 @@ __device__ __forceinline__ f3 composePixel(const float* lg, const float* __restr
 //                       hold two row pairs, and the column pair sits in
 //                       neighbouring lanes;
 //   OUT_APPLY           the 27 used logits stay in LDS and the epilogue runs
-//                       one level of the reconstruction (composePixel: the
+//                       one level of the reconstruction (composePixelStaged: the
 //                       5x5 softmax filter of the level's radiance, blended
 //                       with the coarser output when given; out [h][w][3])
 //                       and writes the error logit (err [h][w]).
@@ -519,12 +443,28 @@ __device__ __forceinline__ void storeApply(const ApplyRegs& r, bool hasCoarse, f
     }
 }
 
+// up(coarse) at tile pixel (lx, ly) from the staged coarser block.  bilinearAxis: coarse pixels a,
+// a + 1 (a = x / 2 for odd x, x / 2 - 1 for even), clamped; in the staged block (first pixel
+// tx*kTS/2 - 1) a sits at (lx + 1) / 2.
+__device__ __forceinline__ f3 upBilinearStaged(const f32x4* co, int lx, int ly) {
+    const int ax = (lx + 1) >> 1, ay = (ly + 1) >> 1;
+    const float wx0 = (lx & 1) ? 0.75f : 0.25f, wy0 = (ly & 1) ? 0.75f : 0.25f;
+    const float wx1 = 1.0f - wx0, wy1 = 1.0f - wy0;
+    auto c = [&](int X, int Y) {
+        const f32x4 v = co[Y * kCoHS + X];
+        return f3{v.x, v.y, v.z};
+    };
+    const f3 top = c(ax, ay) * wx0 + c(ax + 1, ay) * wx1;
+    const f3 bot = c(ax, ay + 1) * wx0 + c(ax + 1, ay + 1) * wx1;
+    return top * wy0 + bot * wy1;
+}
+
 // One level of the reconstruction at tile pixel (lx, ly) from the LDS-staged
 // blocks (one pixel per 16 bytes, rgb in the first three floats): radiance
 // staged with a 2-pixel margin and the coarser output with a 1-pixel margin,
 // both read clamped to their images when staged, so every tap the clamped
 // formula names sits at a constant offset from the pixel's base: the same
-// values, summed in composePixelT's order, with one immediate-offset LDS read
+// values, summed in tap order, with one immediate-offset LDS read
 // per tap and no per-tap index arithmetic.
 __device__ __forceinline__ f3 composePixelStaged(const float* lg, const f32x4* rad, const f32x4* co, bool hasCoarse,
                                                  int lx, int ly) {
@@ -538,19 +478,8 @@ __device__ __forceinline__ f3 composePixelStaged(const float* lg, const f32x4* r
         o = fmaTap(f3{v.x, v.y, v.z}, wgt[j], o);
     }
     if (hasCoarse) {
-        // bilinearAxis: coarse pixels a, a + 1 (a = x / 2 for odd x, x / 2 - 1 for even), clamped;
-        // in the staged block (first pixel tx*kTS/2 - 1) a sits at (lx + 1) / 2
-        const int ax = (lx + 1) >> 1, ay = (ly + 1) >> 1;
-        const float wx0 = (lx & 1) ? 0.75f : 0.25f, wy0 = (ly & 1) ? 0.75f : 0.25f;
-        const float wx1 = 1.0f - wx0, wy1 = 1.0f - wy0;
-        auto c = [&](int X, int Y) {
-            const f32x4 v = co[Y * kCoHS + X];
-            return f3{v.x, v.y, v.z};
-        };
-        const f3 top = c(ax, ay) * wx0 + c(ax + 1, ay) * wx1;
-        const f3 bot = c(ax, ay + 1) * wx0 + c(ax + 1, ay + 1) * wx1;
         const float b = sigmoidf(lg[SGI_KPCN_BLEND_CHANNEL]);
-        o = o + (top * wy0 + bot * wy1 - o) * b;
+        o = o + (upBilinearStaged(co, lx, ly) - o) * b;
     }
     return o;
 }
@@ -1189,69 +1118,136 @@ __global__ void upBackwardKernel(const uint16_t* __restrict__ dout, int H, int W
     *reinterpret_cast<uint4*>(dst) = make_uint4(o[0], o[1], o[2], o[3]);
 }
 
-__global__ void applyKernel(const float* __restrict__ logits, const float* __restrict__ radiance,
-                            const float* __restrict__ coarse, int H, int W, float* __restrict__ out,
-                            float* __restrict__ err) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= W * H) return;
-    const int x = i % W, y = i / W;
-    float lg[28];
-    loadLogits(logits, i, lg);
-    const f3 o = composePixel(lg, radiance, coarse, W, H, x, y);
+// A 16x16 tile of the reconstruction in LDS: its logits (kLogitStride floats per pixel, read from
+// memory as whole lines and not by each pixel's thread, which would touch every line seven times
+// from as many instructions), its radiance with the 5x5 window's margin and its coarser output,
+// both clamped to their images as the taps clamp.
+struct ApplyLds {
+    float4 logits[kTS * kTS * kLogitStride / 4];
+    f32x4 rad[kRadHS * kRadHS];
+    f32x4 co[kCoHS * kCoHS];
+};
+
+__device__ __forceinline__ void stageTile(const float* __restrict__ logits, const float* __restrict__ radiance,
+                                          const float* __restrict__ coarse, int H, int W, int tile, int tilesX,
+                                          ApplyLds& lds) {
+    const int x0 = (tile % tilesX) * kTS, y0 = (tile / tilesX) * kTS;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {  // 16 bytes of a pixel's 32 channels per thread, the last 4 left out
+        const int i = (int)threadIdx.x + k * 256, px = i >> 3, c = i & 7;
+        const int gx = x0 + px % kTS, gy = y0 + px / kTS;
+        if (c < kLogitStride / 4 && gx < W && gy < H)
+            lds.logits[px * (kLogitStride / 4) + c] = reinterpret_cast<const float4*>(logits + ((size_t)gy * W + gx) * kC)[c];
+    }
+    ApplyRegs r;
+    loadApply(radiance, coarse, H, W, tile, tilesX, r);
+    storeApply(r, coarse != nullptr, lds.rad, lds.co);
+    __syncthreads();
+}
+
+__device__ __forceinline__ void tileLogits(const ApplyLds& lds, float* lg) {
+#pragma unroll
+    for (int j = 0; j < kLogitStride / 4; ++j) {
+        const float4 v = lds.logits[threadIdx.x * (kLogitStride / 4) + j];
+        lg[4 * j] = v.x;
+        lg[4 * j + 1] = v.y;
+        lg[4 * j + 2] = v.z;
+        lg[4 * j + 3] = v.w;
+    }
+}
+
+// One level of the reconstruction (1080p: 88 -> 78 us, a thread per pixel over global memory before).
+__global__ __launch_bounds__(256) void applyKernel(const float* __restrict__ logits, const float* __restrict__ radiance,
+                                                   const float* __restrict__ coarse, int H, int W, int tilesX,
+                                                   float* __restrict__ out, float* __restrict__ err) {
+    __shared__ ApplyLds lds;
+    stageTile(logits, radiance, coarse, H, W, blockIdx.x, tilesX, lds);
+    const int lx = (int)threadIdx.x % kTS, ly = (int)threadIdx.x / kTS;
+    const int x = (blockIdx.x % tilesX) * kTS + lx, y = (blockIdx.x / tilesX) * kTS + ly;
+    if (x >= W || y >= H) return;
+    float lg[kLogitStride];
+    tileLogits(lds, lg);
+    const f3 o = composePixelStaged(lg, lds.rad, lds.co, coarse != nullptr, lx, ly);
+    const size_t i = (size_t)y * W + x;
     out[3 * i + 0] = o.x;
     out[3 * i + 1] = o.y;
     out[3 * i + 2] = o.z;
     if (err) err[i] = lg[SGI_KPCN_ERR_CHANNEL];
 }
 
-// Backward of one reconstruction level at pixel i: the logits' gradient
-// (filter taps through the softmax, the blend through the sigmoid, the error
-// channel from derr) and the gradient of up(coarse).
-__global__ void applyBackwardKernel(const float* __restrict__ logits, const float* __restrict__ radiance,
-                                    const float* __restrict__ coarse, const float* __restrict__ dout,
-                                    const float* __restrict__ derr, int H, int W, uint16_t* __restrict__ dlogits,
-                                    float* __restrict__ dup) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= W * H) return;
-    const int x = i % W, y = i / W;
-    float lg[28], wgt[SGI_KPCN_TAPS];
-    loadLogits(logits, i, lg);
-    softmax25(lg, wgt);
-    const f3 g = ld3(dout + 3 * (size_t)i);
-    f3 df = g;
-    float dl[32];
+// Backward of one reconstruction level: the logits' gradient (filter taps
+// through the softmax, the blend through the sigmoid, the error channel from
+// derr) and the gradient of up(coarse).  The tile is staged as the forward's
+// and its gradient leaves through LDS too, as whole lines (1080p: 172 -> 103 us, 4.4 TB/s).
+__global__ __launch_bounds__(256) void applyBackwardKernel(const float* __restrict__ logits,
+                                                           const float* __restrict__ radiance,
+                                                           const float* __restrict__ coarse,
+                                                           const float* __restrict__ dout,
+                                                           const float* __restrict__ derr, int H, int W, int tilesX,
+                                                           uint16_t* __restrict__ dlogits, float* __restrict__ dup) {
+    __shared__ ApplyLds lds;
+    stageTile(logits, radiance, coarse, H, W, blockIdx.x, tilesX, lds);
+    const int lx = (int)threadIdx.x % kTS, ly = (int)threadIdx.x / kTS;
+    const int x0 = (blockIdx.x % tilesX) * kTS, y0 = (blockIdx.x / tilesX) * kTS;
+    const int x = x0 + lx, y = y0 + ly;
+    const bool inside = x < W && y < H;
+    const size_t i = (size_t)y * W + x;
+    float lg[kLogitStride];
+    if (inside) tileLogits(lds, lg);
+    __syncthreads();  // the logits' LDS becomes the gradient's
+    if (inside) {
+        float wgt[SGI_KPCN_TAPS];
+        softmax25(lg, wgt);
+        const f3 g = ld3(dout + 3 * i);
+        f3 df = g;
+        float dl[32];
 #pragma unroll
-    for (int j = 0; j < 32; ++j) dl[j] = 0.0f;
-    if (coarse) {
-        const f3 f = filtered(radiance, W, H, x, y, wgt);
-        const f3 u = upBilinear(coarse, (H + 1) / 2, (W + 1) / 2, x, y);
-        const float b = sigmoidf(lg[SGI_KPCN_BLEND_CHANNEL]);
-        df = g * (1.0f - b);
-        const f3 du = g * b;
-        dup[3 * (size_t)i + 0] = du.x;
-        dup[3 * (size_t)i + 1] = du.y;
-        dup[3 * (size_t)i + 2] = du.z;
-        dl[SGI_KPCN_BLEND_CHANNEL] = dot(g, u - f) * b * (1.0f - b);
+        for (int j = 0; j < 32; ++j) dl[j] = 0.0f;
+        const f32x4* r = lds.rad + ly * kRadHS + lx;  // tap (dx, dy) of the pixel: r[(dy + 2) kRadHS + dx + 2]
+        if (coarse) {
+            f3 f = splat(0.0f);
+#pragma unroll
+            for (int j = 0; j < SGI_KPCN_TAPS; ++j) {
+                const f32x4 v = r[(j / 5) * kRadHS + j % 5];
+                f = fmaTap(f3{v.x, v.y, v.z}, wgt[j], f);
+            }
+            const f3 u = upBilinearStaged(lds.co, lx, ly);
+            const float b = sigmoidf(lg[SGI_KPCN_BLEND_CHANNEL]);
+            df = g * (1.0f - b);
+            const f3 du = g * b;
+            dup[3 * i + 0] = du.x;
+            dup[3 * i + 1] = du.y;
+            dup[3 * i + 2] = du.z;
+            dl[SGI_KPCN_BLEND_CHANNEL] = dot(g, u - f) * b * (1.0f - b);
+        }
+        float dw[SGI_KPCN_TAPS];
+        float sdw = 0.0f;
+#pragma unroll
+        for (int j = 0; j < SGI_KPCN_TAPS; ++j) {
+            const f32x4 v = r[(j / 5) * kRadHS + j % 5];
+            dw[j] = dot(df, f3{v.x, v.y, v.z});
+            sdw += wgt[j] * dw[j];
+        }
+#pragma unroll
+        for (int j = 0; j < SGI_KPCN_TAPS; ++j) dl[j] = wgt[j] * (dw[j] - sdw);
+        if (derr) dl[SGI_KPCN_ERR_CHANNEL] = derr[i];
+        uint4* dst = reinterpret_cast<uint4*>(lds.logits) + threadIdx.x * 5;  // 64 bytes and 16 of padding
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            uint32_t o4[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) o4[j] = f2bf2(dl[q * 8 + 2 * j], dl[q * 8 + 2 * j + 1]);
+            dst[q] = make_uint4(o4[0], o4[1], o4[2], o4[3]);
+        }
     }
-    float dw[SGI_KPCN_TAPS];
-    float sdw = 0.0f;
+    __syncthreads();
 #pragma unroll
-    for (int j = 0; j < SGI_KPCN_TAPS; ++j) {
-        const int xx = min(max(x + j % 5 - 2, 0), W - 1), yy = min(max(y + j / 5 - 2, 0), H - 1);
-        dw[j] = dot(df, ld3(radiance + 3 * ((size_t)yy * W + xx)));
-        sdw += wgt[j] * dw[j];
-    }
-#pragma unroll
-    for (int j = 0; j < SGI_KPCN_TAPS; ++j) dl[j] = wgt[j] * (dw[j] - sdw);
-    if (derr) dl[SGI_KPCN_ERR_CHANNEL] = derr[i];
-    uint4* dst = reinterpret_cast<uint4*>(dlogits + (size_t)i * kC);
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        uint32_t o4[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-            o4[j] = f2bf2(dl[q * 8 + 2 * j], dl[q * 8 + 2 * j + 1]);
-        dst[q] = make_uint4(o4[0], o4[1], o4[2], o4[3]);
+    for (int k = 0; k < 4; ++k) {
+        const int q = (int)threadIdx.x + k * 256, px = q >> 2, c = q & 3;
+        const int gx = x0 + px % kTS, gy = y0 + px / kTS;
+        if (gx < W && gy < H)
+            reinterpret_cast<uint4*>(dlogits + ((size_t)gy * W + gx) * kC)[c] =
+                reinterpret_cast<const uint4*>(lds.logits)[px * 5 + c];
     }
 }
 
@@ -1652,8 +1648,9 @@ hipError_t pyramid(const float* radiance, int H, int W, float* pyr, hipStream_t 
 
 hipError_t applyBackward(const float* logits, const float* radiance, const float* coarse, const float* dout,
                          const float* derr, int H, int W, uint16_t* dlogits, float* dup, hipStream_t s) {
-    hipLaunchKernelGGL(applyBackwardKernel, dim3(gridFor(W * H, 256)), dim3(256), 0, s, logits, radiance, coarse,
-                       dout, derr, H, W, dlogits, dup);
+    const int tilesX = (W + kTS - 1) / kTS, nTiles = tilesX * ((H + kTS - 1) / kTS);
+    hipLaunchKernelGGL(applyBackwardKernel, dim3(nTiles), dim3(256), 0, s, logits, radiance, coarse, dout, derr, H, W,
+                       tilesX, dlogits, dup);
     return hipGetLastError();
 }
 
@@ -1680,8 +1677,8 @@ hipError_t features16Pyramid(const GbufArgs& g, const FrameArgs& fr, const float
 
 hipError_t apply(const float* logits, const float* radiance, const float* coarse, int H, int W, float* out,
                  float* err, hipStream_t s) {
-    hipLaunchKernelGGL(applyKernel, dim3(gridFor(W * H, 256)), dim3(256), 0, s, logits, radiance, coarse, H, W, out,
-                       err);
+    const int tilesX = (W + kTS - 1) / kTS, nTiles = tilesX * ((H + kTS - 1) / kTS);
+    hipLaunchKernelGGL(applyKernel, dim3(nTiles), dim3(256), 0, s, logits, radiance, coarse, H, W, tilesX, out, err);
     return hipGetLastError();
 }
 
