@@ -131,7 +131,8 @@ class Trainer:
         self.dup = [torch.empty((h, w, 3), **f32) for h, w in self.sizes]
         self.derr = torch.empty((height, width), **f32)
         self.partials = torch.empty(int(self.lib.sgi_kpcn_wgrad_partials(height, width)), **f32)
-        self.layer_grad = torch.empty(LAYER_PARAMS, **f32)
+        # one sample's gradient, every layer's slice written by its own launch, added to grad at once
+        self.sample_grad = torch.empty(PARAMS, **f32)
         self.grad = torch.zeros(PARAMS, **f32)
         self.m = torch.zeros(PARAMS, **f32)
         self.v = torch.zeros(PARAMS, **f32)
@@ -187,11 +188,10 @@ class Trainer:
 
     # -- backward ------------------------------------------------------------
     def _layer_back(self, l, x, y, dy, dx_out, level, need_dx=True, stream=0):
-        """Adds layer l's parameter gradient into self.grad; writes the input gradient to dx_out."""
+        """Writes layer l's parameter gradient into self.sample_grad and the input gradient to dx_out."""
         h, w = self.sizes[level]
         _abi.call(self.lib, "sgi_kpcn_conv3x3_wgrad", _p(x), _p(dy), _p(y), h, w, _p(self.partials),
-                  _p(self.layer_grad), stream)
-        self.grad[l * LAYER_PARAMS:(l + 1) * LAYER_PARAMS] += self.layer_grad
+                  self.sample_grad.data_ptr() + 4 * l * LAYER_PARAMS, stream)
         if need_dx:
             _abi.call(self.lib, "sgi_kpcn_conv3x3", _p(dy), _p(y), _p(self.wts.layer_wt(l)), 0, 0, h, w,
                       _p(dx_out), 0, stream)
@@ -243,6 +243,7 @@ class Trainer:
             _abi.call(self.lib, "sgi_kpcn_pool_backward", _p(g[l][0]), h, w, _p(self.gd[l - 1]), 1, stream)
             cur = self.gd[l - 1]
         self._layer_back(0, self.feat, a["e0"], cur, None, 0, need_dx=False, stream=stream)
+        self.grad += self.sample_grad
 
     def zero_grad(self):
         self.grad.zero_()
