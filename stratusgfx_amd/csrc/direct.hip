@@ -24,8 +24,12 @@ __device__ __forceinline__ void directBody(const GbufArgs& g, const FrameArgs& f
     const f3 fragPos = worldPositionFromDepth(texelCentre(x, g.W), texelCentre(y, g.H), g.depth[p], fr.invPV);
     const f3 N = gNormal(g, p);
     const f3 sun = ld3(fr.sunDir);
-    const f3 blends = cascadeBlends(csm, fragPos);
-    const float shadowFactor = infiniteShadowValueBlock(csm, sun, fragPos, blends, N, csm.bias);
+    const f3 L = sun * frsq(dotF(sun, sun));
+    const float NdotLRaw = dotF(N, L);
+    // a surface turned away from the sun reflects exactly 0 of it, whatever the shadow (NaN: tested)
+    float shadowFactor = 0.0f;
+    if (!(NdotLRaw <= 0.0f))
+        shadowFactor = infiniteShadowValueBlock(csm, sun, fragPos, cascadeBlends(csm, fragPos), N, csm.bias);
     // calculateDirectionalLighting passes 1 - shadowFactor, which the Burley path inverts again
     const float sf = 1.0f - (1.0f - shadowFactor);
 
@@ -48,10 +52,9 @@ __device__ __forceinline__ void directBody(const GbufArgs& g, const FrameArgs& f
     const f3 diffuseColor = ((1.0f - metallic) * baseColor) * frcp(1.0f + kEPS);
     const float f0s = 0.16f * reflR * reflR * (1.0f - metallic);
     const f3 f0 = fmaF(baseColor, metallic, splat(f0s));
-    const f3 L = sun * frsq(dotF(sun, sun));
     const f3 VL = V + L;
     const f3 H = VL * frsq(dotF(VL, VL));
-    const float NdotV = saturate(dotF(N, V)), NdotL = saturate(dotF(N, L));
+    const float NdotV = saturate(dotF(N, V)), NdotL = saturate(NdotLRaw);
     const float NdotH = saturate(dotF(N, H)), LdotH = saturate(dotF(L, H));
     // NDF_GGX and Visibility_G_SmithGGX (pbr2.glsl:51-64), Fr_Fresnel_Schlick (:73-76)
     const float r2 = a * a;

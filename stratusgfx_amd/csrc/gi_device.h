@@ -260,52 +260,86 @@ __device__ __forceinline__ f3 cascadeBlends(const CsmArgs& c, f3 p) {
     return f3{b[0], b[1], b[2]};
 }
 
+// Four texels of a row from any texel on (16 bytes, 4-byte aligned).
+typedef float Row4 __attribute__((ext_vector_type(4), aligned(4)));
+
 // One cascade's 9 PCF taps (pbr.glsl:166-174), each the bilinear blend of 4
 // LEQUAL compares, summed in the reference's (y, x) order.  The taps sit one
-// texel apart, so together they cover a 4x4 texel block: the block is read and
-// compared once, and each tap picks its 4 compares from it.  A tap whose
-// rounded floor lands outside the block (its offset rounds across a texel
-// edge) reads its own texels, so the result equals 9 shadowCompare calls.
+// texel apart, so together they cover a 4x4 texel block: the block is read (a
+// row at a time away from the borders) and compared once, and each tap picks
+// its 4 compares from it.  A tap whose rounded floor lands outside the block
+// (its offset rounds across a texel edge) reads its own texels, so the result
+// equals 9 shadowCompare calls.  A block that is all dark or all lit, as most
+// are, needs no picking: the taps are 0, or the sums of their four weights, the
+// same bits.
 __device__ __forceinline__ float pcf9Block(const CsmArgs& c, float s, float t, int layer, float ref) {
     const float* base = c.depth + (size_t)layer * c.res * c.res;
     const float fres = (float)c.res;
     const float wh = 1.0f / fres;
-    const float I0 = floorf((s + -1.0f * wh) * fres - 0.5f);
-    const float J0 = floorf((t + -1.0f * wh) * fres - 0.5f);
-    uint32_t mask = 0;
+    float i0f[3], j0f[3], a[3], b[3];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const size_t row = (size_t)texelIndex(J0 + (float)r, c.res) * c.res;
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-            if (ref <= base[row + texelIndex(I0 + (float)q, c.res)]) mask |= 1u << (r * 4 + q);
+    for (int k = 0; k < 3; ++k) {
+        const float off = (float)(k - 1);
+        const float fu = (s + off * wh) * fres - 0.5f, fv = (t + off * wh) * fres - 0.5f;
+        i0f[k] = floorf(fu);
+        j0f[k] = floorf(fv);
+        a[k] = fu - i0f[k];
+        b[k] = fv - j0f[k];
     }
+    const float I0 = i0f[0], J0 = j0f[0];
+    uint32_t mask = 0;
+    if (I0 >= 0.0f && J0 >= 0.0f && I0 <= fres - 4.0f && J0 <= fres - 4.0f) {
+        const float* q = base + (size_t)(int)J0 * c.res + (int)I0;
+        Row4 row[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) row[r] = *reinterpret_cast<const Row4*>(q + (size_t)r * c.res);
+#pragma unroll
+        for (int k = 0; k < 16; ++k)
+            if (ref <= row[k >> 2][k & 3]) mask |= 1u << k;
+    } else {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const size_t row = (size_t)texelIndex(J0 + (float)r, c.res) * c.res;
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                if (ref <= base[row + texelIndex(I0 + (float)q, c.res)]) mask |= 1u << (r * 4 + q);
+        }
+    }
+    // every tap's texels within the block (false also where a coordinate is not finite)
+    bool within = true;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        const float dq = i0f[k] - I0, dr = j0f[k] - J0;
+        within = within && dq >= 0.0f && dq <= 2.0f && dr >= 0.0f && dr <= 2.0f;
+    }
+    if (within && mask == 0u) return 0.0f;
+    const bool lit = within && mask == 0xFFFFu;
     float light = 0.0f;
 #pragma unroll
-    for (int iy = -1; iy <= 1; ++iy) {
+    for (int iy = 0; iy < 3; ++iy) {
 #pragma unroll
-        for (int ix = -1; ix <= 1; ++ix) {
-            const float x = (float)ix, y = (float)iy;
-            const float fu = (s + x * wh) * fres - 0.5f, fv = (t + y * wh) * fres - 0.5f;
-            const float i0f = floorf(fu), j0f = floorf(fv);
-            const float a = fu - i0f, b = fv - j0f;
-            const float dqf = i0f - I0, drf = j0f - J0;
-            float c00, c10, c01, c11;
-            if (dqf >= 0.0f && dqf <= 2.0f && drf >= 0.0f && drf <= 2.0f) {
-                const int bit = (int)drf * 4 + (int)dqf;
-                c00 = (mask >> bit) & 1u ? 1.0f : 0.0f;
-                c10 = (mask >> (bit + 1)) & 1u ? 1.0f : 0.0f;
-                c01 = (mask >> (bit + 4)) & 1u ? 1.0f : 0.0f;
-                c11 = (mask >> (bit + 5)) & 1u ? 1.0f : 0.0f;
-            } else {
-                const int ia = texelIndex(i0f, c.res), ib = texelIndex(i0f + 1.0f, c.res);
-                const int ja = texelIndex(j0f, c.res), jb = texelIndex(j0f + 1.0f, c.res);
-                c00 = ref <= base[(size_t)ja * c.res + ia] ? 1.0f : 0.0f;
-                c10 = ref <= base[(size_t)ja * c.res + ib] ? 1.0f : 0.0f;
-                c01 = ref <= base[(size_t)jb * c.res + ia] ? 1.0f : 0.0f;
-                c11 = ref <= base[(size_t)jb * c.res + ib] ? 1.0f : 0.0f;
+        for (int ix = 0; ix < 3; ++ix) {
+            const float w00 = (1.0f - a[ix]) * (1.0f - b[iy]), w10 = a[ix] * (1.0f - b[iy]);
+            const float w01 = (1.0f - a[ix]) * b[iy], w11 = a[ix] * b[iy];
+            float c00 = 1.0f, c10 = 1.0f, c01 = 1.0f, c11 = 1.0f;
+            if (!lit) {
+                const float dqf = i0f[ix] - I0, drf = j0f[iy] - J0;
+                if (dqf >= 0.0f && dqf <= 2.0f && drf >= 0.0f && drf <= 2.0f) {
+                    const int bit = (int)drf * 4 + (int)dqf;
+                    c00 = (mask >> bit) & 1u ? 1.0f : 0.0f;
+                    c10 = (mask >> (bit + 1)) & 1u ? 1.0f : 0.0f;
+                    c01 = (mask >> (bit + 4)) & 1u ? 1.0f : 0.0f;
+                    c11 = (mask >> (bit + 5)) & 1u ? 1.0f : 0.0f;
+                } else {
+                    const int ia = texelIndex(i0f[ix], c.res), ib = texelIndex(i0f[ix] + 1.0f, c.res);
+                    const int ja = texelIndex(j0f[iy], c.res), jb = texelIndex(j0f[iy] + 1.0f, c.res);
+                    c00 = ref <= base[(size_t)ja * c.res + ia] ? 1.0f : 0.0f;
+                    c10 = ref <= base[(size_t)ja * c.res + ib] ? 1.0f : 0.0f;
+                    c01 = ref <= base[(size_t)jb * c.res + ia] ? 1.0f : 0.0f;
+                    c11 = ref <= base[(size_t)jb * c.res + ib] ? 1.0f : 0.0f;
+                }
             }
-            light += (1.0f - a) * (1.0f - b) * c00 + a * (1.0f - b) * c10 + (1.0f - a) * b * c01 + a * b * c11;
+            light += w00 * c00 + w10 * c10 + w01 * c01 + w11 * c11;
         }
     }
     return light;
@@ -313,23 +347,30 @@ __device__ __forceinline__ float pcf9Block(const CsmArgs& c, float s, float t, i
 
 // pbr.glsl:158-227 calculateInfiniteShadowValue with the block-read PCF (the
 // 9 taps of each of the two cascades from one 4x4 texel block: the same value
-// as 36 single compares); `bias` already zero when unused.
+// as 36 single compares); `bias` already zero when unused.  Where the blend's
+// weight is exactly 0 or 1 (all but the bands where cascades meet) the other
+// cascade's taps are multiplied by 0 and left out.
 __device__ __forceinline__ float infiniteShadowValueBlock(const CsmArgs& c, f3 sunDir, f3 fragPos, f3 blends, f3 normal,
                                                           float bias) {
     const f3 position = fragPos + normal * (1.0f - saturate(dot(normal, sunDir))) * 1.0f;
     const bool beyond2 = blends.y >= 0.0f, beyond3 = blends.z >= 0.0f;
-    const int index1 = beyond2 ? 2 : 0, index2 = beyond3 ? 3 : 1;
-    float c1[4], c2[4];
-    mulMat4(c.projViews[index1], position.x, position.y, position.z, 1.0f, c1);
-    mulMat4(c.projViews[index2], position.x, position.y, position.z, 1.0f, c2);
-    const float s1 = (c1[0] / c1[3]) * 0.5f + 0.5f, t1 = (c1[1] / c1[3]) * 0.5f + 0.5f;
-    const float depth1 = (c1[2] / c1[3]) * 0.5f + 0.5f;
-    const float s2 = (c2[0] / c2[3]) * 0.5f + 0.5f, t2 = (c2[1] / c2[3]) * 0.5f + 0.5f;
-    float depth2 = (c2[2] / c2[3]) * 0.5f + 0.5f;
-    depth2 = beyond3 ? saturate(depth2) : depth2;
     const float weight = beyond2 ? saturate(blends.y) - saturate(blends.z) : 1.0f - saturate(blends.x);
-    const float light1 = pcf9Block(c, s1, t1, index1, depth1 - bias);
-    const float light2 = pcf9Block(c, s2, t2, index2, depth2 - bias);
+    float light1 = 0.0f, light2 = 0.0f;
+    if (weight != 0.0f) {
+        const int index = beyond2 ? 2 : 0;
+        float h[4];
+        mulMat4(c.projViews[index], position.x, position.y, position.z, 1.0f, h);
+        const float depth = (h[2] / h[3]) * 0.5f + 0.5f;
+        light1 = pcf9Block(c, (h[0] / h[3]) * 0.5f + 0.5f, (h[1] / h[3]) * 0.5f + 0.5f, index, depth - bias);
+    }
+    if (weight != 1.0f) {
+        const int index = beyond3 ? 3 : 1;
+        float h[4];
+        mulMat4(c.projViews[index], position.x, position.y, position.z, 1.0f, h);
+        float depth = (h[2] / h[3]) * 0.5f + 0.5f;
+        depth = beyond3 ? saturate(depth) : depth;
+        light2 = pcf9Block(c, (h[0] / h[3]) * 0.5f + 0.5f, (h[1] / h[3]) * 0.5f + 0.5f, index, depth - bias);
+    }
     return mixv(light2, light1, weight) * (1.0f / 9.0f);
 }
 
