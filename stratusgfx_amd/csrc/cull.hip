@@ -355,8 +355,8 @@ __global__ __launch_bounds__(64) void cullTilesKernel(GbufArgs g, FrameArgs fr, 
                                                       int32_t* __restrict__ tiles) {
     __shared__ float comp[cullLdsFloats<TS>()];
     __shared__ float sums[6];
-    cullTileBody<TS>(g, fr, (int)xcdSwizzle(blockIdx.x, (uint32_t)nTiles), tilesX, K, vpls, visible, remap, stage1,
-                     tiles, comp, sums);
+    const int t = (int)xcdSpread(blockIdx.x);
+    if (t < nTiles) cullTileBody<TS>(g, fr, t, tilesX, K, vpls, visible, remap, stage1, tiles, comp, sums);
 }
 
 // Batched: the tiles of every view, numbered view after view.
@@ -365,7 +365,8 @@ __global__ __launch_bounds__(64) void cullTilesViewsKernel(const sgi_batch::View
                                                            int numViews, int totalTiles, int K) {
     __shared__ float comp[cullLdsFloats<TS>()];
     __shared__ float sums[6];
-    const int gt = (int)xcdSwizzle(blockIdx.x, (uint32_t)totalTiles);
+    const int gt = (int)xcdSpread(blockIdx.x);
+    if (gt >= totalTiles) return;
     const sgi_batch::ViewDesc& d = views[sgi_batch::findView<sgi_batch::kTiles>(views, numViews, gt)];
     cullTileBody<TS>(d.g, d.fr, gt - d.tileStart, d.tilesX, K, d.vplUpdated, d.visible, 0, nullptr, d.tiles, comp,
                      sums);
@@ -399,15 +400,15 @@ hipError_t cullTiles(const GbufArgs& g, const FrameArgs& fr, int tileSize, int t
     const int nTiles = tilesX * tilesY;
     switch (tileSize) {
         case 8:
-            hipLaunchKernelGGL(cullTilesKernel<8>, dim3(nTiles), dim3(64), 0, s, g, fr, tilesX, nTiles, K, vpls,
+            hipLaunchKernelGGL(cullTilesKernel<8>, dim3(spreadBlocks(nTiles)), dim3(64), 0, s, g, fr, tilesX, nTiles, K, vpls,
                                visible, remap, stage1, tiles);
             break;
         case 16:
-            hipLaunchKernelGGL(cullTilesKernel<16>, dim3(nTiles), dim3(64), 0, s, g, fr, tilesX, nTiles, K, vpls,
+            hipLaunchKernelGGL(cullTilesKernel<16>, dim3(spreadBlocks(nTiles)), dim3(64), 0, s, g, fr, tilesX, nTiles, K, vpls,
                                visible, remap, stage1, tiles);
             break;
         case 32:
-            hipLaunchKernelGGL(cullTilesKernel<32>, dim3(nTiles), dim3(64), 0, s, g, fr, tilesX, nTiles, K, vpls,
+            hipLaunchKernelGGL(cullTilesKernel<32>, dim3(spreadBlocks(nTiles)), dim3(64), 0, s, g, fr, tilesX, nTiles, K, vpls,
                                visible, remap, stage1, tiles);
             break;
         default:
@@ -458,14 +459,14 @@ hipError_t cullTilesViews(const sgi_batch::ViewDesc* views, int numViews, int to
                           hipStream_t s) {
     switch (tileSize) {
         case 8:
-            hipLaunchKernelGGL(cullTilesViewsKernel<8>, dim3(totalTiles), dim3(64), 0, s, views, numViews, totalTiles, K);
+            hipLaunchKernelGGL(cullTilesViewsKernel<8>, dim3(spreadBlocks(totalTiles)), dim3(64), 0, s, views, numViews, totalTiles, K);
             break;
         case 16:
-            hipLaunchKernelGGL(cullTilesViewsKernel<16>, dim3(totalTiles), dim3(64), 0, s, views, numViews, totalTiles,
+            hipLaunchKernelGGL(cullTilesViewsKernel<16>, dim3(spreadBlocks(totalTiles)), dim3(64), 0, s, views, numViews, totalTiles,
                                K);
             break;
         case 32:
-            hipLaunchKernelGGL(cullTilesViewsKernel<32>, dim3(totalTiles), dim3(64), 0, s, views, numViews, totalTiles,
+            hipLaunchKernelGGL(cullTilesViewsKernel<32>, dim3(spreadBlocks(totalTiles)), dim3(64), 0, s, views, numViews, totalTiles,
                                K);
             break;
         default:

@@ -2,7 +2,7 @@
 // and no point lights: 3x3 PCF over two blended cascades
 // (calculateInfiniteShadowValue, pbr.glsl:158-227) times BRDF_Burley
 // (pbr2.glsl:194-250) through calculateLighting_Burley (pbr2.glsl:454-478).
-// One thread per pixel; blocks cover 16x16 tiles, XCD-contiguous.  Not built
+// One thread per pixel; blocks cover 16x16 tiles, in chunks per XCD.  Not built
 // with the exact-contraction rule of the other passes where it says so below:
 // only the shading after the shadow factor is contracted.
 #include "launch.h"
@@ -85,13 +85,15 @@ __device__ __forceinline__ void directBody(const GbufArgs& g, const FrameArgs& f
 
 __global__ __launch_bounds__(256) void directKernel(GbufArgs g, FrameArgs fr, CsmArgs csm, int tilesX, int nTiles,
                                                     float* __restrict__ lit) {
-    directBody(g, fr, csm, (int)xcdSwizzle(blockIdx.x, (uint32_t)nTiles), tilesX, lit);
+    const int t = (int)xcdSpread(blockIdx.x);
+    if (t < nTiles) directBody(g, fr, csm, t, tilesX, lit);
 }
 
 // Batched: the 16x16 tiles of every view, numbered view after view.
 __global__ __launch_bounds__(256) void directViewsKernel(const sgi_batch::ViewDesc* __restrict__ views, int numViews,
                                                          int total) {
-    const int gt = (int)xcdSwizzle(blockIdx.x, (uint32_t)total);
+    const int gt = (int)xcdSpread(blockIdx.x);
+    if (gt >= total) return;
     const sgi_batch::ViewDesc& d = views[sgi_batch::findView<sgi_batch::kDirectTiles>(views, numViews, gt)];
     directBody(d.g, d.fr, d.csm, gt - d.dtileStart, (d.g.W + 15) / 16, d.direct);
 }
@@ -102,12 +104,12 @@ namespace sgi_launch {
 
 hipError_t directLight(const GbufArgs& g, const FrameArgs& fr, const CsmArgs& csm, float* lit, hipStream_t s) {
     const int tx = (g.W + 15) / 16, ty = (g.H + 15) / 16;
-    hipLaunchKernelGGL(directKernel, dim3(tx * ty), dim3(256), 0, s, g, fr, csm, tx, tx * ty, lit);
+    hipLaunchKernelGGL(directKernel, dim3(spreadBlocks(tx * ty)), dim3(256), 0, s, g, fr, csm, tx, tx * ty, lit);
     return hipGetLastError();
 }
 
 hipError_t directLightViews(const sgi_batch::ViewDesc* views, int numViews, int totalTiles16, hipStream_t s) {
-    hipLaunchKernelGGL(directViewsKernel, dim3(totalTiles16), dim3(256), 0, s, views, numViews, totalTiles16);
+    hipLaunchKernelGGL(directViewsKernel, dim3(spreadBlocks(totalTiles16)), dim3(256), 0, s, views, numViews, totalTiles16);
     return hipGetLastError();
 }
 

@@ -1,8 +1,8 @@
 // Per-pixel VPL gather — vpl_pbr_gi.fs:81-207.
 //
 // One 256-thread block shades one 16x16 screen tile (blocks are mapped to
-// tiles XCD-contiguously so that neighbouring tiles, which fetch the same VPL
-// cube texels, share an L2).  In tile-list mode the tile's list of up to K VPL
+// tiles in chunks per XCD, so that neighbouring tiles, which fetch the same VPL
+// cube texels, share an L2 and every XCD gets its share of the costly ones).  In tile-list mode the tile's list of up to K VPL
 // records and atlas entries is staged once into LDS and every lane walks it
 // with broadcast LDS reads; in the reference's random mode each pixel hashes
 // its own VPL slots and reads the records through the cache hierarchy.
@@ -474,8 +474,9 @@ __global__ __launch_bounds__(TS * TS) void gatherTilesKernel(GbufArgs g, FrameAr
                                                             float* __restrict__ color, float* __restrict__ reservoir) {
     __shared__ Vpl lv[kMaxK];
     __shared__ int ln;
-    gatherTileBody<FMT, TS, HALF>(g, fr, cubes, (int)xcdSwizzle(blockIdx.x, (uint32_t)nTiles), tilesX, K, vpls,
-                                  entries, tiles, color, reservoir, lv, ln);
+    const uint32_t t = xcdSpread(blockIdx.x);
+    if (t >= (uint32_t)nTiles) return;
+    gatherTileBody<FMT, TS, HALF>(g, fr, cubes, (int)t, tilesX, K, vpls, entries, tiles, color, reservoir, lv, ln);
 }
 
 // Batched: the tiles of every view, numbered view after view (FP32 shading).
@@ -484,7 +485,8 @@ __global__ __launch_bounds__(TS * TS) void gatherTilesViewsKernel(const sgi_batc
                                                                  int numViews, int totalTiles, int K, CubeArgs cubes) {
     __shared__ Vpl lv[kMaxK];
     __shared__ int ln;
-    const int gt = (int)xcdSwizzle(blockIdx.x, (uint32_t)totalTiles);
+    const int gt = (int)xcdSpread(blockIdx.x);
+    if (gt >= totalTiles) return;
     const sgi_batch::ViewDesc& d = views[sgi_batch::findView<sgi_batch::kTiles>(views, numViews, gt)];
     gatherTileBody<FMT, TS, false>(d.g, d.fr, cubes, gt - d.tileStart, d.tilesX, K, d.vplUpdated, d.entries, d.tiles,
                                    d.color, d.reservoir, lv, ln);
@@ -513,7 +515,8 @@ __global__ __launch_bounds__(256) void gatherRandomKernel(GbufArgs g, FrameArgs 
                                                          int nTiles, const PackedVpl* __restrict__ prep,
                                                          const int32_t* __restrict__ visible,
                                                          float* __restrict__ color, float* __restrict__ reservoir) {
-    const uint32_t t = xcdSwizzle(blockIdx.x, (uint32_t)nTiles);
+    const uint32_t t = xcdSpread(blockIdx.x);
+    if (t >= (uint32_t)nTiles) return;
     const int tx = (int)t % tilesX, ty = (int)t / tilesX;
     const int x = tx * 16 + (int)threadIdx.x % 16, y = ty * 16 + (int)threadIdx.x / 16;
     if (x >= g.W || y >= g.H) return;
@@ -581,7 +584,8 @@ __global__ __launch_bounds__(256) void gatherAllKernel(GbufArgs g, FrameArgs fr,
                                                       const sgi_atlas_entry* __restrict__ entries,
                                                       float* __restrict__ color, float* __restrict__ reservoir) {
     __shared__ Vpl lv[256];
-    const uint32_t t = xcdSwizzle(blockIdx.x, (uint32_t)nTiles);
+    const uint32_t t = xcdSpread(blockIdx.x);
+    if (t >= (uint32_t)nTiles) return;
     const int tx = (int)t % tilesX, ty = (int)t / tilesX;
     const int x = tx * 16 + (int)threadIdx.x % 16, y = ty * 16 + (int)threadIdx.x / 16;
     const bool inside = x < g.W && y < g.H;
@@ -632,7 +636,8 @@ __global__ __launch_bounds__(256) void gatherSamplesKernel(GbufArgs g, FrameArgs
                                                           const PackedVpl* __restrict__ prep,
                                                           const int32_t* __restrict__ visible,
                                                           float* __restrict__ color, float* __restrict__ reservoir) {
-    const uint32_t t = xcdSwizzle(blockIdx.x, (uint32_t)nTiles);
+    const uint32_t t = xcdSpread(blockIdx.x);
+    if (t >= (uint32_t)nTiles) return;
     const int tx = (int)t % tilesX, ty = (int)t / tilesX;
     const int x = tx * 16 + (int)threadIdx.x % 16, y = ty * 16 + (int)threadIdx.x / 16;
     if (x >= g.W || y >= g.H) return;
@@ -724,7 +729,8 @@ __global__ __launch_bounds__(256) void gatherSamplesCompactKernel(GbufArgs g, Fr
     __shared__ float4 lit[4][64];                    // a pair's lighting and its factor
     __shared__ float rew[4][64];                     // a pair's reweighting factor
     const int lane = (int)threadIdx.x & 63, wave = (int)threadIdx.x >> 6;
-    const uint32_t t = xcdSwizzle(blockIdx.x, (uint32_t)nTiles);
+    const uint32_t t = xcdSpread(blockIdx.x);
+    if (t >= (uint32_t)nTiles) return;
     const int tx = (int)t % tilesX, ty = (int)t / tilesX;
     const int x = tx * 16 + (int)threadIdx.x % 16, y = ty * 16 + (int)threadIdx.x / 16;
     const bool live = x < g.W && y < g.H;
@@ -834,22 +840,22 @@ hipError_t launchEx(const GbufArgs& g, const FrameArgs& fr, const CubeArgs& cube
     const int rx = (g.W + 15) / 16, ry = (g.H + 15) / 16;
     if (mode == SGI_GATHER_ALL) {
         if (accumulate64)
-            hipLaunchKernelGGL((gatherAllKernel<FMT, true>), dim3(rx * ry), dim3(256), 0, s, g, fr, cubes, rx, rx * ry,
+            hipLaunchKernelGGL((gatherAllKernel<FMT, true>), dim3(spreadBlocks(rx * ry)), dim3(256), 0, s, g, fr, cubes, rx, rx * ry,
                                vpls, visible, entries, color, reservoir);
         else
-            hipLaunchKernelGGL((gatherAllKernel<FMT, false>), dim3(rx * ry), dim3(256), 0, s, g, fr, cubes, rx,
+            hipLaunchKernelGGL((gatherAllKernel<FMT, false>), dim3(spreadBlocks(rx * ry)), dim3(256), 0, s, g, fr, cubes, rx,
                                rx * ry, vpls, visible, entries, color, reservoir);
     } else {
         const hipError_t e = prepare<FMT>(cubes, vpls, visible, entries, prep, s);
         if (e != hipSuccess) return e;
         if (half)
-            hipLaunchKernelGGL((gatherSamplesKernel<FMT, true>), dim3(rx * ry), dim3(256), 0, s, g, fr, cubes, rx,
+            hipLaunchKernelGGL((gatherSamplesKernel<FMT, true>), dim3(spreadBlocks(rx * ry)), dim3(256), 0, s, g, fr, cubes, rx,
                                rx * ry, samples, rejectionLimit, prep, visible, color, reservoir);
         else if (rejectionLimit < 0)
-            hipLaunchKernelGGL((gatherSamplesCompactKernel<FMT>), dim3(rx * ry), dim3(256), 0, s, g, fr, cubes, rx,
+            hipLaunchKernelGGL((gatherSamplesCompactKernel<FMT>), dim3(spreadBlocks(rx * ry)), dim3(256), 0, s, g, fr, cubes, rx,
                                rx * ry, samples, prep, halfPositions(prep), visible, color, reservoir);
         else
-            hipLaunchKernelGGL((gatherSamplesKernel<FMT, false>), dim3(rx * ry), dim3(256), 0, s, g, fr, cubes, rx,
+            hipLaunchKernelGGL((gatherSamplesKernel<FMT, false>), dim3(spreadBlocks(rx * ry)), dim3(256), 0, s, g, fr, cubes, rx,
                                rx * ry, samples, rejectionLimit, prep, visible, color, reservoir);
     }
     return hipGetLastError();
@@ -863,22 +869,22 @@ hipError_t launchFmt(const GbufArgs& g, const FrameArgs& fr, const CubeArgs& cub
         const int rx = (g.W + 15) / 16, ry = (g.H + 15) / 16;
         const hipError_t e = prepare<FMT>(cubes, vpls, visible, entries, prep, s);
         if (e != hipSuccess) return e;
-        hipLaunchKernelGGL((gatherRandomKernel<FMT, HALF>), dim3(rx * ry), dim3(256), 0, s, g, fr, cubes, rx, rx * ry,
+        hipLaunchKernelGGL((gatherRandomKernel<FMT, HALF>), dim3(spreadBlocks(rx * ry)), dim3(256), 0, s, g, fr, cubes, rx, rx * ry,
                            prep, visible, color, reservoir);
         return hipGetLastError();
     }
     const int nTiles = tilesX * tilesY;
     switch (tileSize) {
         case 8:
-            hipLaunchKernelGGL((gatherTilesKernel<FMT, 8, HALF>), dim3(nTiles), dim3(64), 0, s, g, fr, cubes, tilesX,
+            hipLaunchKernelGGL((gatherTilesKernel<FMT, 8, HALF>), dim3(spreadBlocks(nTiles)), dim3(64), 0, s, g, fr, cubes, tilesX,
                                nTiles, K, vpls, entries, tiles, color, reservoir);
             break;
         case 16:
-            hipLaunchKernelGGL((gatherTilesKernel<FMT, 16, HALF>), dim3(nTiles), dim3(256), 0, s, g, fr, cubes, tilesX,
+            hipLaunchKernelGGL((gatherTilesKernel<FMT, 16, HALF>), dim3(spreadBlocks(nTiles)), dim3(256), 0, s, g, fr, cubes, tilesX,
                                nTiles, K, vpls, entries, tiles, color, reservoir);
             break;
         case 32:
-            hipLaunchKernelGGL((gatherTilesKernel<FMT, 32, HALF>), dim3(nTiles), dim3(1024), 0, s, g, fr, cubes,
+            hipLaunchKernelGGL((gatherTilesKernel<FMT, 32, HALF>), dim3(spreadBlocks(nTiles)), dim3(1024), 0, s, g, fr, cubes,
                                tilesX, nTiles, K, vpls, entries, tiles, color, reservoir);
             break;
         default:
@@ -938,7 +944,7 @@ hipError_t gatherViews(const sgi_batch::ViewDesc* views, int numViews, int total
                        const CubeArgs& cubes, int format, hipStream_t s) {
     const int threads = tileSize * tileSize;
 #define SGI_GATHER_VIEWS(F, T)                                                                                      \
-    hipLaunchKernelGGL((gatherTilesViewsKernel<F, T>), dim3(totalTiles), dim3(threads), 0, s, views, numViews,     \
+    hipLaunchKernelGGL((gatherTilesViewsKernel<F, T>), dim3(spreadBlocks(totalTiles)), dim3(threads), 0, s, views, numViews,     \
                        totalTiles, K, cubes)
     if (format == SGI_TEXEL_F16) {
         if (tileSize == 8) SGI_GATHER_VIEWS(SGI_TEXEL_F16, 8);

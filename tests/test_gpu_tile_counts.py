@@ -1,0 +1,62 @@
+"""Frames of 1, 127, 128, 129 and 8 x 17 tiles of 16 x 16: the blocks of the gathers, tile culling and
+direct light are dealt to the XCDs in chunks of 16 tiles, so a launch holds up to 127 blocks without a
+tile.  Every tile has to be done once, and nothing written beyond the last one."""
+import numpy as np
+import pytest
+
+import oracle as orc
+from gpu_util import Case, assert_tiles_equal, require_gpu, small
+from stratusgfx_amd import _abi
+from stratusgfx_amd import scene as sc
+from stratusgfx_amd.gi import GiPass
+
+pytestmark = pytest.mark.gpu
+
+REL_L2 = 1e-4  # FP32 images, the bound of every parity test
+
+
+@pytest.mark.parametrize("W,H", [(16, 16), (2032, 16), (1024, 32), (2049, 7), (125, 270)])
+def test_every_tile_once(W, H):
+    torch = require_gpu()
+    case = Case(small(sc.CORNELL_640x360, name=f"cornell-{W}x{H}-24vpl", width=W, height=H, num_vpls=24,
+                      cube_res=32, csm_res=256))
+    ts, K = 16, 7
+    gi = GiPass(W, H, ts, K)
+    gi.set_frame(case.dev.frame)
+    gi.set_csm(case.dev.csm_struct())
+    upd, vis, ent = case.oracle_cull()
+    d_upd, d_vis = torch.from_numpy(upd).cuda(), torch.from_numpy(vis).cuda()
+    d_ent = torch.from_numpy(np.ascontiguousarray(ent)).cuda()
+    g = case.dev.gbuffer()
+
+    def images():  # the frame's rows and one row more, which stays as it is
+        return [torch.full((H + 1, W, c), 7.0, dtype=torch.float32, device="cuda") for c in (3, 4)]
+
+    def check(got, want):
+        torch.cuda.synchronize()
+        for a, b in zip(got, want):
+            assert orc.rel_l2(a[:H].cpu().numpy(), b) <= REL_L2
+            assert bool((a[H] == 7.0).all())
+
+    _, o_tiles = orc.cull_tiles(case.host.frame, case.hg, ts, K, upd, vis)
+    tiles = torch.full((gi.num_tiles + 1, 1 + K), -5, dtype=torch.int32, device="cuda")
+    gi.cull_tiles(g, d_upd, d_vis, tiles[:gi.num_tiles])
+    torch.cuda.synchronize()
+    assert_tiles_equal(tiles[:gi.num_tiles].cpu().numpy(), o_tiles)
+    assert bool((tiles[gi.num_tiles] == -5).all())
+
+    args = (case.host.frame, case.hg, upd, int(vis[0]), ent, case.hcubes)
+    col, res = images()
+    gi.gather(g, d_upd, d_vis, d_ent, case.dev.cubes(), tiles[:gi.num_tiles], col[:H], res[:H])
+    check((col, res), orc.gather(*args, tiles=o_tiles, tile_size=ts, K=K, mode=orc.GATHER_TILES))
+    col, res = images()
+    gi.gather(g, d_upd, d_vis, d_ent, case.dev.cubes(), None, col[:H], res[:H])
+    check((col, res), orc.gather(*args, mode=orc.GATHER_RANDOM))
+    for mode, omode, kw in ((_abi.GATHER_ALL, orc.GATHER_CONVERGED, {}),
+                            (_abi.GATHER_SAMPLES, orc.GATHER_SAMPLES, dict(samples=4, rejection_limit=5))):
+        col, res = images()
+        gi.gather_ex(g, d_upd, d_vis, d_ent, case.dev.cubes(), None, col[:H], res[:H], mode=mode, **kw)
+        check((col, res), orc.gather(*args, mode=omode, precision=0, **kw))
+    lit = images()[0]
+    gi.direct_light(g, lit[:H])
+    check((lit,), (orc.direct_light(case.host.frame, case.hcsm, case.hg),))
