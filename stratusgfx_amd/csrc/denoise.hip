@@ -12,7 +12,7 @@
 //           denoiseTemporalKernel: the temporal blend with the reprojected
 //           history and the combine screen + albedo * gi.
 //
-// Blocks cover 64x4 pixels and are numbered so that each XCD walks a
+// Blocks cover 64x4 pixels (the filter: eight rows spread over 64x32) and are numbered so that each XCD walks a
 // contiguous band of rows: the 5x5 taps at stride 8 reach 16 rows up and down,
 // and that window stays in the XCD's L2 instead of being fetched once per XCD.
 // The edge-stopping weights and the normalisation are continuous, so they use
@@ -153,6 +153,12 @@ __global__ __launch_bounds__(256) void denoiseMergeViewsKernel(const sgi_batch::
     mergeBody(d.g, d.fr, d.visible, (const float4*)d.reservoir, d.resA, d.normals, x, y);
 }
 
+// filterInput, vpl_pbr_gi_denoise.fs:142-190: the weight of a tap with normal and depth n for a centre with c
+__device__ __forceinline__ float filterWeight(const float4& c, const float4& n) {
+    const float wz = fexp(-fabsf(c.w - n.w));
+    return pow128(gmax(0.0f, dotF(f3{c.x, c.y, c.z}, f3{n.x, n.y, n.z}))) * wz;
+}
+
 __device__ __forceinline__ void filterBody(const GbufArgs& g, int stride, const float4* __restrict__ resIn,
                                            const float4* __restrict__ normals, float4* __restrict__ resOut, int x,
                                            int y) {
@@ -160,8 +166,6 @@ __device__ __forceinline__ void filterBody(const GbufArgs& g, int stride, const 
     const int W = g.W, H = g.H;
     const size_t p = (size_t)y * W + x;
     const float4 cn4 = normals[p];
-    const f3 centerNormal = f3{cn4.x, cn4.y, cn4.z};
-    const float centerDepth = cn4.w;
     float rf0 = 0.0f, rf1 = 0.0f, rf2 = 0.0f, rf3 = 0.0f;
 #pragma unroll
     for (int dx = -2; dx <= 2; ++dx) {
@@ -171,16 +175,7 @@ __device__ __forceinline__ void filterBody(const GbufArgs& g, int stride, const 
             const int ty = clampx(y + dy * stride, H);
             const size_t q = (size_t)ty * W + tx;
             const float4 rr = resIn[q];
-            float filtered;
-            if (dx == 0 && dy == 0) {
-                filtered = 1.0f;
-            } else {  // filterInput, vpl_pbr_gi_denoise.fs:142-190
-                const float4 n4 = normals[q];
-                const float wz = fexp(-fabsf(centerDepth - n4.w));
-                float wn = gmax(0.0f, dotF(centerNormal, f3{n4.x, n4.y, n4.z}));
-                wn = pow128(wn);
-                filtered = wn * wz;
-            }
+            const float filtered = dx == 0 && dy == 0 ? 1.0f : filterWeight(cn4, normals[q]);
             rf0 = __builtin_fmaf(filtered, rr.x, rf0);
             rf1 = __builtin_fmaf(filtered, rr.y, rf1);
             rf2 = __builtin_fmaf(filtered, rr.z, rf2);
@@ -191,12 +186,76 @@ __device__ __forceinline__ void filterBody(const GbufArgs& g, int stride, const 
     resOut[p] = make_float4(rf0 * inv, rf1 * inv, rf2 * inv, 1.0f);
 }
 
-__global__ __launch_bounds__(256) void denoiseFilterKernel(GbufArgs g, int stride, const float4* __restrict__ resIn,
+// The same sums, in the same order, for four pixels of a column: rows y0, y0 + S, y0 + 2 S, y0 + 3 S of
+// column x lie on one lattice of the pass, so their taps are 5 x 8 texels and not 4 x 25, and y0 is the
+// same over the wave, so a tap's row costs no vector address.  One pixel per thread was bound by the
+// 800 B a pixel read through L1 (62 us a pass at 1080p, vector ALU 56 % busy); this form takes 40, 40 and
+// 50 us at strides 2, 4 and 8, against 12 us for the bytes and about 30 for the arithmetic.  The columns
+// of taps stay a loop: unrolled, their loads are hoisted and 350 registers leave one wave per SIMD.
+template <int S>
+__device__ __forceinline__ void filterColumn(const GbufArgs& g, const float4* __restrict__ resIn,
+                                             const float4* __restrict__ normals, float4* __restrict__ resOut, int x,
+                                             int y0) {
+    const int W = g.W, H = g.H;
+    const int xc = x < W ? x : W - 1;
+    const float4* nRow[8];
+    const float4* rRow[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const size_t o = (size_t)clampx(y0 + (j - 2) * S, H) * W;
+        nRow[j] = normals + o;
+        rRow[j] = resIn + o;
+    }
+    float4 cn[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) cn[k] = nRow[k + 2][xc];
+    float rf[4][4] = {};
+#pragma unroll 1
+    for (int dx = -2; dx <= 2; ++dx) {
+        const int tx = clampx(xc + dx * S, W);
+        float4 n[8], r[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            n[j] = nRow[j][tx];
+            r[j] = rRow[j][tx];
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+#pragma unroll
+            for (int dy = -2; dy <= 2; ++dy) {
+                const int j = k + 2 + dy;
+                const float f = dx == 0 && dy == 0 ? 1.0f : filterWeight(cn[k], n[j]);
+                rf[k][0] = __builtin_fmaf(f, r[j].x, rf[k][0]);
+                rf[k][1] = __builtin_fmaf(f, r[j].y, rf[k][1]);
+                rf[k][2] = __builtin_fmaf(f, r[j].z, rf[k][2]);
+                rf[k][3] = __builtin_fmaf(f, r[j].w, rf[k][3]);
+            }
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const int y = y0 + k * S;
+        if (x >= W || y >= H) continue;
+        const float inv = frcp(gmax(kEPS, rf[k][3]));
+        resOut[(size_t)y * W + x] = make_float4(rf[k][0] * inv, rf[k][1] * inv, rf[k][2] * inv, 1.0f);
+    }
+}
+
+// 64 x 32 pixel regions, eight waves each in two blocks: wave w of a region starts at row
+// (w / S) 4 S + w % S, so S waves cover 4 S rows.
+template <int S>
+__device__ __forceinline__ void filterRegion(const GbufArgs& g, const float4* __restrict__ resIn,
+                                             const float4* __restrict__ normals, float4* __restrict__ resOut, int b) {
+    const int regionsX = (g.W + 63) / 64, r = b >> 1;
+    const int w = __builtin_amdgcn_readfirstlane((b & 1) * 4 + (int)(threadIdx.x >> 6));
+    const int y0 = (r / regionsX) * 32 + (w / S) * 4 * S + w % S;
+    filterColumn<S>(g, resIn, normals, resOut, (r % regionsX) * 64 + (int)(threadIdx.x & 63), y0);
+}
+
+template <int S>
+__global__ __launch_bounds__(256) void denoiseFilterKernel(GbufArgs g, const float4* __restrict__ resIn,
                                                            const float4* __restrict__ normals,
                                                            float4* __restrict__ resOut) {
-    int x, y;
-    blockPixel(g.W, g.H, x, y);
-    filterBody(g, stride, resIn, normals, resOut, x, y);
+    filterRegion<S>(g, resIn, normals, resOut, (int)xcdSwizzle(blockIdx.x, gridDim.x));
 }
 
 __global__ __launch_bounds__(256) void denoiseFilterListKernel(GbufArgs g, int stride, const float4* __restrict__ resIn,
@@ -206,14 +265,15 @@ __global__ __launch_bounds__(256) void denoiseFilterListKernel(GbufArgs g, int s
     forListedTiles(list, g.W, [&](int x, int y) { filterBody(g, stride, resIn, normals, resOut, x, y); });
 }
 
-// pass 1: resA -> resB, pass 2: resB -> resA, pass 3: resA -> reservoirOut
+// pass 1: resA -> resB, pass 2: resB -> resA, pass 3: resA -> reservoirOut; region blocks in view order
+template <int PASS>
 __global__ __launch_bounds__(256) void denoiseFilterViewsKernel(const sgi_batch::ViewDesc* __restrict__ views,
-                                                                int numViews, int total, int pass) {
-    int x, y;
-    const sgi_batch::ViewDesc& d = viewBlock(views, numViews, total, x, y);
-    const float4* in = pass == 2 ? d.resB : d.resA;
-    float4* out = pass == 1 ? d.resB : (pass == 2 ? d.resA : (float4*)d.reservoirOut);
-    filterBody(d.g, 1 << pass, in, d.normals, out, x, y);
+                                                                int numViews) {
+    const int b = (int)xcdSwizzle(blockIdx.x, gridDim.x);
+    const sgi_batch::ViewDesc& d = views[sgi_batch::findView<sgi_batch::kFilterBlocks>(views, numViews, b)];
+    const float4* in = PASS == 2 ? d.resB : d.resA;
+    float4* out = PASS == 1 ? d.resB : (PASS == 2 ? d.resA : (float4*)d.reservoirOut);
+    filterRegion<1 << PASS>(d.g, in, d.normals, out, b - d.dfilterStart);
 }
 
 // The final pass's temporal blend and combine (vpl_pbr_gi_denoise.fs:336-434) on
@@ -410,16 +470,19 @@ hipError_t denoiseSpatial(const GbufArgs& cur, const FrameArgs& fr, const int32_
     if (e != hipSuccess || mergeOnly) return e;
     float4* const in[3] = {ws.resA, ws.resB, ws.resA};
     float4* const out[3] = {ws.resB, ws.resA, (float4*)reservoirOut};
-    for (int pass = 0; pass < 3 && e == hipSuccess; ++pass) {
-        if (tiles)
+    if (tiles) {
+        for (int pass = 0; pass < 3 && e == hipSuccess; ++pass) {
             hipLaunchKernelGGL(denoiseFilterListKernel, lgrid, block, 0, s, cur, 2 << pass, in[pass], ws.normals,
                                out[pass], tiles);
-        else
-            hipLaunchKernelGGL(denoiseFilterKernel, grid, block, 0, s, cur, 2 << pass, in[pass], ws.normals,
-                               out[pass]);
-        e = hipGetLastError();
+            e = hipGetLastError();
+        }
+        return e;
     }
-    return e;
+    const dim3 fgrid(sgi_batch::filterBlocks(cur.W, cur.H));
+    hipLaunchKernelGGL(denoiseFilterKernel<2>, fgrid, block, 0, s, cur, in[0], ws.normals, out[0]);
+    hipLaunchKernelGGL(denoiseFilterKernel<4>, fgrid, block, 0, s, cur, in[1], ws.normals, out[1]);
+    hipLaunchKernelGGL(denoiseFilterKernel<8>, fgrid, block, 0, s, cur, in[2], ws.normals, out[2]);
+    return hipGetLastError();
 }
 
 hipError_t denoiseTemporal(const GbufArgs& cur, const GbufArgs& prev, const FrameArgs& fr, const float* screen,
@@ -451,14 +514,15 @@ hipError_t denoise(const GbufArgs& cur, const GbufArgs& prev, const FrameArgs& f
                            historyOut, ws, s);
 }
 
-hipError_t denoiseViews(const sgi_batch::ViewDesc* views, int numViews, int totalBlocks, hipStream_t s) {
+hipError_t denoiseViews(const sgi_batch::ViewDesc* views, int numViews, int totalBlocks, int totalFilter,
+                        hipStream_t s) {
     hipLaunchKernelGGL(denoiseMergeViewsKernel, dim3(totalBlocks), dim3(256), 0, s, views, numViews, totalBlocks);
     hipError_t e = hipGetLastError();
-    for (int pass = 1; pass <= 3 && e == hipSuccess; ++pass) {
-        hipLaunchKernelGGL(denoiseFilterViewsKernel, dim3(totalBlocks), dim3(256), 0, s, views, numViews, totalBlocks,
-                           pass);
-        e = hipGetLastError();
-    }
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(denoiseFilterViewsKernel<1>, dim3(totalFilter), dim3(256), 0, s, views, numViews);
+    hipLaunchKernelGGL(denoiseFilterViewsKernel<2>, dim3(totalFilter), dim3(256), 0, s, views, numViews);
+    hipLaunchKernelGGL(denoiseFilterViewsKernel<3>, dim3(totalFilter), dim3(256), 0, s, views, numViews);
+    e = hipGetLastError();
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(denoiseTemporalViewsKernel, dim3(totalBlocks), dim3(256), 0, s, views, numViews, totalBlocks);
     return hipGetLastError();

@@ -97,7 +97,8 @@ hipError_t cullTilesViews(const sgi_batch::ViewDesc* views, int numViews, int to
 hipError_t gatherViews(const sgi_batch::ViewDesc* views, int numViews, int totalTiles, int tileSize, int K,
                        const sgi_dev::CubeArgs& cubes, int format, hipStream_t s);
 hipError_t directLightViews(const sgi_batch::ViewDesc* views, int numViews, int totalTiles16, hipStream_t s);
-hipError_t denoiseViews(const sgi_batch::ViewDesc* views, int numViews, int totalBlocks, hipStream_t s);
+hipError_t denoiseViews(const sgi_batch::ViewDesc* views, int numViews, int totalBlocks, int totalFilter,
+                        hipStream_t s);
 
 // The merge and the three filter passes into reservoirOut; tiles (a device
 // list of 16x16 tiles: int32 count, then tile indices; NULL = the whole

@@ -19,6 +19,7 @@ struct ViewDesc {
     int tileStart;       // first batch tile of this view
     int dtileStart;      // first batch 16x16 tile (direct light)
     int dblockStart;     // first batch 64x4 block (denoiser)
+    int dfilterStart;    // first batch block of the denoiser's filter (filterBlocks() a view)
     sgi_vpl* vplUpdated;
     int32_t* visible;
     sgi_atlas_entry* entries;
@@ -38,14 +39,20 @@ struct ViewDesc {
     float4* normals;
 };
 
-enum Offset { kTiles = 0, kDirectTiles = 1, kDenoiseBlocks = 2 };
+enum Offset { kTiles = 0, kDirectTiles = 1, kDenoiseBlocks = 2, kFilterBlocks = 3 };
+
+// Blocks of one a-trous filter launch over a W x H view: two for each region of 64 x 32 pixels.
+__host__ __device__ __forceinline__ int filterBlocks(int W, int H) { return ((W + 63) / 64) * ((H + 31) / 32) * 2; }
 
 // The view whose work items contain batch item `item` (views are in item order).
 template <int OFF>
 __device__ __forceinline__ int findView(const ViewDesc* __restrict__ v, int n, int item) {
     int i = 0;
     for (int k = 1; k < n; ++k) {
-        const int start = OFF == kTiles ? v[k].tileStart : (OFF == kDirectTiles ? v[k].dtileStart : v[k].dblockStart);
+        const int start = OFF == kTiles         ? v[k].tileStart
+                          : OFF == kDirectTiles ? v[k].dtileStart
+                          : OFF == kFilterBlocks ? v[k].dfilterStart
+                                                 : v[k].dblockStart;
         if (start <= item) i = k;
     }
     return i;

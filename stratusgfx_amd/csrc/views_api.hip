@@ -19,7 +19,7 @@ void sgi_set_error(const std::string& msg);
 struct sgi_views {
     sgi_views_config cfg{};
     int device = 0;
-    int numViews = 0, totalTiles = 0, totalTiles16 = 0, totalBlocks = 0, numVpls = 0, maxEntries = 0;
+    int numViews = 0, totalTiles = 0, totalTiles16 = 0, totalBlocks = 0, totalFilter = 0, numVpls = 0, maxEntries = 0;
     const sgi_vpl* vpls = nullptr;
     const sgi_atlas_entry* shadowIndices = nullptr;
     sgi_dev::CubeArgs cubes{};
@@ -46,7 +46,7 @@ struct sgi_views {
     hipGraphExec_t exec = nullptr;
     // what the captured launches baked in (grid sizes and by-value arguments)
     struct Shape {
-        int numViews, totalTiles, totalTiles16, totalBlocks, numVpls, cubeFormat;
+        int numViews, totalTiles, totalTiles16, totalBlocks, totalFilter, numVpls, cubeFormat;
         const sgi_vpl* vpls;
         const sgi_atlas_entry* shadowIndices;
         sgi_dev::CubeArgs cubes;
@@ -95,6 +95,7 @@ sgi_views::Shape shapeOf(const sgi_views* v) {
     s.totalTiles = v->totalTiles;
     s.totalTiles16 = v->totalTiles16;
     s.totalBlocks = v->totalBlocks;
+    s.totalFilter = v->totalFilter;
     s.numVpls = v->numVpls;
     s.cubeFormat = v->cubeFormat;
     s.vpls = v->vpls;
@@ -110,7 +111,8 @@ sgi_views::Shape shapeOf(const sgi_views* v) {
 
 bool sameShape(const sgi_views::Shape& a, const sgi_views::Shape& b) {
     bool same = a.numViews == b.numViews && a.totalTiles == b.totalTiles && a.totalTiles16 == b.totalTiles16 &&
-                a.totalBlocks == b.totalBlocks && a.numVpls == b.numVpls && a.cubeFormat == b.cubeFormat &&
+                a.totalBlocks == b.totalBlocks && a.totalFilter == b.totalFilter &&
+                a.numVpls == b.numVpls && a.cubeFormat == b.cubeFormat &&
                 a.vpls == b.vpls && a.shadowIndices == b.shadowIndices && a.cubes.numAtlases == b.cubes.numAtlases &&
                 a.cubes.res == b.cubes.res && a.cubes.layers == b.cubes.layers;
     for (int i = 0; same && i < SGI_MAX_TOTAL_SHADOW_ATLASES; ++i) same = a.cubes.atlas[i] == b.cubes.atlas[i];
@@ -160,7 +162,7 @@ hipError_t runStages(sgi_views* v, hipStream_t s) {
     if (e == hipSuccess)
         e = sgi_launch::gatherViews(v->descs, v->numViews, v->totalTiles, c.tile_size, c.max_vpls_per_tile, v->cubes,
                                     v->cubeFormat, s);
-    if (e == hipSuccess) e = sgi_launch::denoiseViews(v->descs, v->numViews, v->totalBlocks, s);
+    if (e == hipSuccess) e = sgi_launch::denoiseViews(v->descs, v->numViews, v->totalBlocks, v->totalFilter, s);
     return e;
 }
 
@@ -243,7 +245,7 @@ int sgi_views_set(sgi_views* v, int32_t numViews, const sgi_view_io* io, const s
 
     const int ts = v->cfg.tile_size, cap = SGI_MAX_TOTAL_VPLS_PER_FRAME;
     int64_t pix = 0;
-    int tiles = 0, tiles16 = 0, blocks = 0;
+    int tiles = 0, tiles16 = 0, blocks = 0, filter = 0;
     for (int i = 0; i < numViews; ++i) {
         const sgi_view_io& x = io[i];
         const sgi_gbuffer& g = x.gbuffer;
@@ -274,9 +276,11 @@ int sgi_views_set(sgi_views* v, int32_t numViews, const sgi_view_io* io, const s
         d.tileStart = tiles;
         d.dtileStart = tiles16;
         d.dblockStart = blocks;
+        d.dfilterStart = filter;
         tiles += d.tilesX * d.tilesY;
         tiles16 += ((g.width + 15) / 16) * ((g.height + 15) / 16);
         blocks += ((g.width + 63) / 64) * ((g.height + 3) / 4);
+        filter += sgi_batch::filterBlocks(g.width, g.height);
         d.vplUpdated = v->vplUpdated + (size_t)i * cap;
         d.visible = v->visible + (size_t)i * (1 + cap);
         d.entries = v->entries + (size_t)i * cap;
@@ -313,6 +317,7 @@ int sgi_views_set(sgi_views* v, int32_t numViews, const sgi_view_io* io, const s
     v->totalTiles = tiles;
     v->totalTiles16 = tiles16;
     v->totalBlocks = blocks;
+    v->totalFilter = filter;
     v->numVpls = numVpls;
     v->maxEntries = numVpls < cap ? numVpls : cap;
     v->vpls = vpls;
