@@ -221,11 +221,9 @@ __device__ __forceinline__ bool visibility(const Pixel& px, const FrameArgs& fr,
     const float distanceRatio = clampv((2.0f * dist) * L.invRadius, 0.0f, 1.0f);
     float shadowFactor = 0.0f;
     if (px.distToCamera < 500.0f) {  // calculateShadowValue1Sample, pbr.glsl:116-136
-        const f3 fragDir = px.P - L.pos;
-        // bias = |P - L| * max(minBias, saturate(dot(L - P, N)) * 0.03); dot(L - P, N)
-        // has the same products in the same order as dot(N, L - P)
-        const float m = gmax(0.1f, saturate(nl) * 0.03f);
-        const float depth = cubeFetch<FMT>(L.cube, cubes.res, fragDir) * L.farPlane;
+        // bias = |P - L| * max(0.1, saturate(dot(L - P, N)) * 0.03): the second is at most 0.03
+        const float m = 0.1f;
+        const float depth = cubeFetch<FMT>(L.cube, cubes.res, lmf * -1.0f) * L.farPlane;
         const float lhs = dist - dist * m;
         bool shadowed;
         if (__builtin_expect(fabsf(lhs - depth) > dist * 0x1p-18f, 1))

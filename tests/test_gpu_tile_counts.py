@@ -1,6 +1,7 @@
 """Frames of 1, 127, 128, 129 and 8 x 17 tiles of 16 x 16: the blocks of the gathers, tile culling and
 direct light are dealt to the XCDs in chunks of 16 tiles, so a launch holds up to 127 blocks without a
-tile.  Every tile has to be done once, and nothing written beyond the last one."""
+tile.  Every tile has to be done once, and nothing written beyond the last one.  The cubes are of even, odd and
+unit size: a lookup near a texel's edge takes the exact formula, any other an estimate."""
 import numpy as np
 import pytest
 
@@ -15,11 +16,11 @@ pytestmark = pytest.mark.gpu
 REL_L2 = 1e-4  # FP32 images, the bound of every parity test
 
 
-@pytest.mark.parametrize("W,H", [(16, 16), (2032, 16), (1024, 32), (2049, 7), (125, 270)])
-def test_every_tile_once(W, H):
+@pytest.mark.parametrize("W,H,cube", [(16, 16, 1), (2032, 16, 32), (1024, 32, 31), (2049, 7, 32), (125, 270, 7)])
+def test_every_tile_once(W, H, cube):
     torch = require_gpu()
     case = Case(small(sc.CORNELL_640x360, name=f"cornell-{W}x{H}-24vpl", width=W, height=H, num_vpls=24,
-                      cube_res=32, csm_res=256))
+                      cube_res=cube, csm_res=256))
     ts, K = 16, 7
     gi = GiPass(W, H, ts, K)
     gi.set_frame(case.dev.frame)
