@@ -572,9 +572,58 @@ __global__ __launch_bounds__(256) void gatherRandomKernel(GbufArgs g, FrameArgs 
     writeOut(g, p, vplColor, validSamples, color, reservoir);
 }
 
+// A wave's pixels around one of them, for a test that rejects a VPL for all of them at once: the pixel's
+// position and normal, the largest |N_i - Nc|, the largest N_i . (Pc - P_i) and the largest |P_i - Pc|.
+// The converged gather runs it over every VPL, a VPL per lane: at 1080p with 4096 lights it drops more than
+// half of them for a wave and the pass takes 12.3 ms instead of 13.3.  A tile's list holds the lights near
+// its means, and dropping the few left in it costs what it saves (493 against 496 us).
+struct WaveBounds {
+    f3 Pc, Nc;
+    float spread, lift, extent;
+    bool ok;  // every position and normal is finite
+};
+
+__device__ __forceinline__ float waveMax(float v) {
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
+    return v;
+}
+
+// The whole wave calls it; live: this lane has a pixel.
+__device__ __forceinline__ WaveBounds waveBounds(const Pixel& px, bool live) {
+    WaveBounds b;
+    const uint64_t alive = __ballot(live);
+    const int c = alive >> 40 & 1u ? 40 : __ffsll((unsigned long long)alive) - 1;  // (row 2, column 8) of 16 x 4
+    const auto from = [&](float v) {
+        return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), c < 0 ? 0 : c));
+    };
+    b.Pc = f3{from(px.P.x), from(px.P.y), from(px.P.z)};
+    b.Nc = f3{from(px.N.x), from(px.N.y), from(px.N.z)};
+    const f3 dN = px.N - b.Nc, dP = b.Pc - px.P;
+    const float spread = fsqrt(dotF(dN, dN)), extent = fsqrt(dotF(dP, dP)), lift = dotF(px.N, dP);
+    // NaN and infinity fail the comparison
+    b.ok = __ballot(live && !(spread < 4.0f && extent < 1e18f && fabsf(lift) < 1e18f)) == 0;
+    b.spread = waveMax(live ? spread : 0.0f);
+    b.extent = waveMax(live ? extent : 0.0f);
+    b.lift = waveMax(live ? lift : -1e18f);
+    return b;
+}
+
+// Whether passesSideRadius may accept the VPL for one of the wave's pixels.  With D = L - Pc,
+// N_i . (L - P_i) = Nc . D + (N_i - Nc) . D + N_i . (Pc - P_i) <= Nc . D + spread |D| + lift and
+// |L - P_i| >= |D| - extent; a VPL is dropped only where these clear 2^-12 of the lengths involved, far
+// above the rounding of the test it stands for, so every pixel would have rejected it.  A NaN keeps it.
+__device__ __forceinline__ bool waveMayPass(const WaveBounds& b, f3 pos, float radius) {
+    const f3 D = pos - b.Pc;
+    const float d = fsqrt(dotF(D, D)), margin = 0x1p-12f * (d + b.extent);
+    const bool behind = __builtin_fmaf(b.spread, d, dotF(b.Nc, D)) + b.lift < -margin;
+    const bool beyond = d - b.extent > __builtin_fmaf(radius, 1.0f + 0x1p-12f, margin);
+    return !(b.ok && (behind || beyond));
+}
+
 // Every visible VPL per pixel (the converged estimate), optionally summed in
-// FP64.  The VPLs are staged through LDS 256 at a time and every lane of the
-// 16x16 tile walks the chunk.
+// FP64.  The VPLs are staged through LDS 256 at a time and every wave of the
+// 16x16 tile walks those that one of its pixels may accept, in their order.
 template <int FMT, bool ACC64>
 __global__ __launch_bounds__(256) void gatherAllKernel(GbufArgs g, FrameArgs fr, CubeArgs cubes, int tilesX,
                                                       int nTiles, const sgi_vpl* __restrict__ vpls,
@@ -588,8 +637,10 @@ __global__ __launch_bounds__(256) void gatherAllKernel(GbufArgs g, FrameArgs fr,
     const int x = tx * 16 + (int)threadIdx.x % 16, y = ty * 16 + (int)threadIdx.x / 16;
     const bool inside = x < g.W && y < g.H;
     const size_t p = inside ? (size_t)y * g.W + x : 0;
-    Pixel px;
+    Pixel px{};
     if (inside) px = setupPixel(g, fr, x, y, p);
+    const WaveBounds wb = waveBounds(px, inside);
+    const int lane = (int)threadIdx.x & 63;
     const int count = min(max(visible[0], 0), SGI_MAX_TOTAL_VPLS_PER_FRAME);
     double c64[4] = {0.0, 0.0, 0.0, 0.0};
     f3 vplColor = splat(0.0f);
@@ -599,19 +650,24 @@ __global__ __launch_bounds__(256) void gatherAllKernel(GbufArgs g, FrameArgs fr,
         __syncthreads();
         if ((int)threadIdx.x < n) lv[threadIdx.x] = loadVpl<FMT>(vpls + base + threadIdx.x, entries + base + threadIdx.x, cubes);
         __syncthreads();
-        if (!inside) continue;
-        for (int k = 0; k < n; ++k) {
-            if (ACC64) {
-                f3 c = splat(0.0f);
-                float w = 0.0f;
-                if (evalVpl<FMT>(px, fr, cubes, lv[k], true, c, w)) {
-                    c64[0] += (double)c.x;
-                    c64[1] += (double)c.y;
-                    c64[2] += (double)c.z;
-                    c64[3] += (double)w;
+        for (int k0 = 0; k0 < n; k0 += 64) {
+            const int mine = min(k0 + lane, n - 1);
+            uint64_t keep = __ballot(k0 + lane < n && waveMayPass(wb, lv[mine].pos, lv[mine].radius));
+            if (!inside) continue;
+            for (; keep; keep &= keep - 1) {
+                const Vpl& L = lv[k0 + __ffsll((unsigned long long)keep) - 1];
+                if (ACC64) {
+                    f3 c = splat(0.0f);
+                    float w = 0.0f;
+                    if (evalVpl<FMT>(px, fr, cubes, L, true, c, w)) {
+                        c64[0] += (double)c.x;
+                        c64[1] += (double)c.y;
+                        c64[2] += (double)c.z;
+                        c64[3] += (double)w;
+                    }
+                } else {
+                    evalVpl<FMT>(px, fr, cubes, L, true, vplColor, validSamples);
                 }
-            } else {
-                evalVpl<FMT>(px, fr, cubes, lv[k], true, vplColor, validSamples);
             }
         }
     }

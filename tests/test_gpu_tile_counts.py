@@ -61,3 +61,32 @@ def test_every_tile_once(W, H, cube):
     lit = images()[0]
     gi.direct_light(g, lit[:H])
     check((lit,), (orc.direct_light(case.host.frame, case.hcsm, case.hg),))
+
+
+@pytest.mark.parametrize("radius", [None, 0.5, 6.0, 1.0e6])
+@pytest.mark.parametrize("accumulate_fp64", [False, True])
+def test_converged_drops_only_rejected(radius, accumulate_fp64):
+    """The converged gather drops a VPL for a whole wave where none of its pixels can accept it: radii as
+    generated, small enough to drop nearly all, about a tile's extent, and without end."""
+    torch = require_gpu()
+    W, H = 200, 75
+    case = Case(small(sc.CORNELL_640x360, name="cornell-200x75-90vpl", width=W, height=H, num_vpls=90, cube_res=16,
+                      csm_res=64))
+    gi = GiPass(W, H, 16, 12)
+    gi.set_frame(case.dev.frame)
+    gi.set_csm(case.dev.csm_struct())
+    upd, vis, ent = case.oracle_cull()
+    if radius is not None:
+        upd = upd.copy()
+        upd[:, 12] = radius
+    d = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()  # noqa: E731
+    col = torch.zeros((H, W, 3), dtype=torch.float32, device="cuda")
+    res = torch.zeros((H, W, 4), dtype=torch.float32, device="cuda")
+    gi.gather_ex(case.dev.gbuffer(), d(upd), d(vis), d(ent), case.dev.cubes(), None, col, res, mode=_abi.GATHER_ALL,
+                 accumulate_fp64=accumulate_fp64)
+    torch.cuda.synchronize()
+    oc, orr = orc.gather(case.host.frame, case.hg, upd, int(vis[0]), ent, case.hcubes, mode=orc.GATHER_CONVERGED,
+                         precision=0)
+    assert orc.rel_l2(res.cpu().numpy(), orr) <= REL_L2
+    assert float(np.abs(res[..., 3].cpu().numpy().astype(np.float64) - orr[..., 3]).max()) < 1e-3
+    assert orc.rel_l2(col.cpu().numpy(), oc) <= REL_L2
