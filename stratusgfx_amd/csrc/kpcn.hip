@@ -390,7 +390,6 @@ constexpr int kLogitStride = 28;
 constexpr int kRadHS = kTS + 4;     // radiance staged for the 5x5 taps (OUT_APPLY)
 constexpr int kCoHS = kTS / 2 + 2;  // the coarser output staged for up() (OUT_APPLY)
 constexpr int kRadSlots = (kRadHS * kRadHS + 255) / 256;  // staged pixels per thread
-constexpr int kCoSlots = (kCoHS * kCoHS + 255) / 256;
 
 // OUT_APPLY's blocks of one tile, loaded into registers one tile ahead and
 // stored to LDS at the tile's start: its radiance (2-pixel margin, kRadHS^2
@@ -498,23 +497,44 @@ struct MfmaOp<ACT_F8> {
 // output (OUT_BF16 / OUT_BF16_POOL) is stored in. When either is FP8 the epilogue
 // is scaled: bias holds [k1[32], k2[32]] and a channel's value is fma(acc, k1, k2)
 // (otherwise acc + bias).
-// Blocks resident per CU: two (VGPRs near 256, and for OUT_APPLY the staged blocks in LDS),
-// three for FP8 inputs on the plain path (FP8 weights take 36 VGPRs instead of 72 and the
-// FP8 halo 15.5 KB of LDS; the deferred up-add's raw chunks would not fit the 168 VGPRs)
-// and for the first convolution with its weights in LDS.
-// The first convolution (BF16, 16-channel features in) keeps its weight fragments in
-// LDS, one copy per block (9 taps x 2 channel blocks x 64 lanes x 16 B = 18 KB), each
-// wave reading a tap's two fragments before its MFMAs: without the 72 VGPRs they take in
-// registers it runs three blocks per CU (75 -> 72 us at 1080p). On the other layers the
-// extra LDS round trip before the first MFMA cost more than the third block gave.
-template <int IN, int AIN>
+// Blocks resident per CU: two where the weight fragments sit in registers as BF16 (72 VGPRs, near 256 in
+// all), else three.  FP8 weights take 36, and the reconstruction's FP8 form keeps them in LDS, as does the
+// first convolution (BF16, 16-channel features in): one copy per block (9 taps x 2 channel blocks x 64
+// lanes), each wave reading a tap's two fragments before its MFMAs.  The first convolution 75 -> 72 us at
+// 1080p; at 4K in FP8 the level-0 reconstruction 347 -> 314 us, the deferred up-add 56 -> 52.  On the
+// other BF16 layers the extra LDS round trip before the first MFMA cost more than the third block gave.
+template <int IN, int OUT, int AIN>
 constexpr bool weightsInLds() {
-    return AIN == ACT_BF16 && IN == IN_PLAIN16;
+    return AIN == ACT_BF16 ? IN == IN_PLAIN16 : OUT == OUT_APPLY;
 }
 
 template <int IN, int OUT, int AIN>
 constexpr int convBlocksPerCu() {
-    return OUT != OUT_APPLY && ((AIN == ACT_F8 && IN == IN_PLAIN) || weightsInLds<IN, AIN>()) ? 3 : 2;
+    return AIN == ACT_F8 || weightsInLds<IN, OUT, AIN>() ? 3 : 2;
+}
+
+// Stores a lane's channels 8 lg .. 8 lg + 7 of pixel p.
+template <int AOUT>
+__device__ __forceinline__ void storeChannels(void* out, size_t p, int lg, const uint32_t* bits) {
+    char* const q = static_cast<char*>(out) + p * Act<AOUT>::kPixBytes;
+    if constexpr (AOUT == ACT_F8)
+        *reinterpret_cast<uint2*>(q + 8 * lg) = make_uint2(bits[0], bits[1]);
+    else
+        *reinterpret_cast<uint4*>(q + 16 * lg) = make_uint4(bits[0], bits[1], bits[2], bits[3]);
+}
+
+// The output channel in row m of MFMA block mb.  A lane ends up with rows 4 lg .. 4 lg + 3 of both blocks;
+// for a stored activation they are made eight neighbouring channels, so that a lane stores 16 bytes of
+// BF16 (8 of FP8) at once and a wave whole lines, instead of a half of every pixel twice (the first
+// convolution with its pooling 73 -> 66 us at 1080p, with FP8 output at 4K 255 -> 225).
+template <int OUT>
+__device__ __forceinline__ constexpr int convChannel(int mb, int m) {
+    return OUT == OUT_BF16 || OUT == OUT_BF16_POOL ? (m >> 2) * 8 + mb * 4 + (m & 3) : mb * 16 + m;
+}
+
+// lane l ^ 1's value (a quad permute, no LDS)
+__device__ __forceinline__ float columnNeighbour(float v) {
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xB1, 0xF, 0xF, true));
 }
 
 template <int IN, int OUT, int AIN, int AOUT>
@@ -527,36 +547,40 @@ __global__ __launch_bounds__(256, (convBlocksPerCu<IN, OUT, AIN>())) void conv3x
     constexpr int kLogitU4 = kTS * kTS * kLogitStride / 4;
     constexpr int kSmemU4 = OUT == OUT_APPLY && kLogitU4 > kHaloU4 ? kLogitU4 : kHaloU4;
     __shared__ uint4 smem[kSmemU4];  // the input halo, then (OUT_APPLY) the tile's logits
-    __shared__ f32x4 radS[OUT == OUT_APPLY ? kRadSlots * 256 : 1];
-    __shared__ f32x4 coS[OUT == OUT_APPLY ? kCoSlots * 256 : 1];
+    __shared__ f32x4 radS[OUT == OUT_APPLY ? kRadHS * kRadHS : 1];
+    __shared__ f32x4 coS[OUT == OUT_APPLY ? kCoHS * kCoHS : 1];
     // IN_UPADD with OUT_APPLY: the coarser operand staged by stageUp (the
     // epilogue needs the registers a deferred add would hold)
     constexpr bool kLdsUp = IN == IN_UPADD && OUT == OUT_APPLY;
     constexpr bool kDefer = IN == IN_UPADD && !kLdsUp;
     constexpr int kHaloIn = kLdsUp ? IN_PLAIN : IN;  // the skip operand loads as a plain input
     __shared__ uint4 upS[IN == IN_UPADD && OUT == OUT_APPLY ? UpStage<AIN>::kSlots * 256 : 1];
-    constexpr bool kWLds = weightsInLds<IN, AIN>();
-    __shared__ uint4 wS[kWLds ? 9 * 2 * 64 : 1];  // fragment (t, mb) of lane l at (2 t + mb) 64 + l
+    constexpr bool kWLds = weightsInLds<IN, OUT, AIN>();
+    typedef typename MfmaOp<AIN>::T Frag;
+    __shared__ Frag wS[kWLds ? 9 * 2 * 64 : 1];  // fragment (t, mb) of lane l at (2 t + mb) 64 + l
     constexpr bool kFlags = IN == IN_UPADD && OUT == OUT_APPLY;
     __shared__ float flagS[kFlags ? 256 : 1];  // the tile's exp(min(err, 80)), pixel by pixel
     uint4* halo = smem;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int l16 = lane & 15, lg = lane >> 4;
     // A operands: W[t][mb*16 + l16][8 lg .. 8 lg + 7]
-    typename MfmaOp<AIN>::T wa[kWLds ? 1 : 9][2];
+    Frag wa[kWLds ? 1 : 9][2];
     if constexpr (kWLds) {
         // visible to every wave after the first tile's barriers, before its first MFMA
         for (int i = (int)threadIdx.x; i < 9 * 2 * 64; i += 256) {
             const int t = i >> 7, mb = (i >> 6) & 1, ln = i & 63;
-            const size_t e = (size_t)(t * kC + mb * 16 + (ln & 15)) * kC + 8 * (ln >> 4);
-            wS[i] = *reinterpret_cast<const uint4*>(static_cast<const uint16_t*>(w) + e);
+            const size_t e = (size_t)(t * kC + convChannel<OUT>(mb, ln & 15)) * kC + 8 * (ln >> 4);
+            if constexpr (AIN == ACT_F8)
+                wS[i] = *reinterpret_cast<const long*>(static_cast<const uint8_t*>(w) + e);
+            else
+                wS[i] = asBf16x8(*reinterpret_cast<const uint4*>(static_cast<const uint16_t*>(w) + e));
         }
     } else {
 #pragma unroll
         for (int t = 0; t < 9; ++t)
 #pragma unroll
             for (int mb = 0; mb < 2; ++mb) {
-                const size_t e = (size_t)(t * kC + mb * 16 + l16) * kC + 8 * lg;
+                const size_t e = (size_t)(t * kC + convChannel<OUT>(mb, l16)) * kC + 8 * lg;
                 if constexpr (AIN == ACT_F8)
                     wa[t][mb] = *reinterpret_cast<const long*>(static_cast<const uint8_t*>(w) + e);
                 else
@@ -568,7 +592,7 @@ __global__ __launch_bounds__(256, (convBlocksPerCu<IN, OUT, AIN>())) void conv3x
     for (int mb = 0; mb < 2; ++mb)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            const int o = mb * 16 + 4 * lg + r;
+            const int o = convChannel<OUT>(mb, 4 * lg + r);
             k1v[mb][r] = kScaled ? bias[o] : 1.0f;
             bv[mb][r] = kScaled ? bias[kC + o] : (bias ? bias[o] : 0.0f);
         }
@@ -623,12 +647,11 @@ __global__ __launch_bounds__(256, (convBlocksPerCu<IN, OUT, AIN>())) void conv3x
                     halo[px * A::kPxU4 + c] = addChunkT<AIN>(pre[k], preB[k]);
                 } else if constexpr (kLdsUp) {
                     // in-image halo pixels add their coarser pixel; the zero padding stays zero
-                    const int gy = ty * kTS - 1 + px / kHS, gx = tx * kTS - 1 + px % kHS;
+                    const int dy = px / kHS, dx = px % kHS;
+                    const int gy = ty * kTS - 1 + dy, gx = tx * kTS - 1 + dx;
                     uint4 v = pre[k];
-                    if (gx >= 0 && gx < W && gy >= 0 && gy < H) {
-                        const int q = ((gy >> 1) - (ty * (kTS / 2) - 1)) * kUpHS + (gx >> 1) - (tx * (kTS / 2) - 1);
-                        v = addChunkT<AIN>(v, upS[q * A::kChunks + c]);
-                    }
+                    if (gx >= 0 && gx < W && gy >= 0 && gy < H)  // its coarser pixel's place is the thread's own
+                        v = addChunkT<AIN>(v, upS[(((dy + 1) >> 1) * kUpHS + ((dx + 1) >> 1)) * A::kChunks + c]);
                     halo[px * A::kPxU4 + c] = v;
                 } else {
                     halo[px * A::kPxU4 + c] = pre[k];
@@ -658,10 +681,10 @@ __global__ __launch_bounds__(256, (convBlocksPerCu<IN, OUT, AIN>())) void conv3x
 #pragma unroll
         for (int t = 0; t < 9; ++t) {
             const int dy = t / 3, dx = t % 3;
-            typename MfmaOp<AIN>::T a0, a1;
+            Frag a0, a1;
             if constexpr (kWLds) {
-                a0 = ldsBf16x8(wS + (2 * t) * 64 + lane);
-                a1 = ldsBf16x8(wS + (2 * t + 1) * 64 + lane);
+                a0 = wS[(2 * t) * 64 + lane];
+                a1 = wS[(2 * t + 1) * 64 + lane];
             } else {
                 a0 = wa[t][0];
                 a1 = wa[t][1];
@@ -742,6 +765,7 @@ __global__ __launch_bounds__(256, (convBlocksPerCu<IN, OUT, AIN>())) void conv3x
             for (int nb = 0; nb < 4; ++nb) {
                 const int y = ty * kTS + wave * 4 + nb;
                 const size_t p = (size_t)y * W + x;
+                uint32_t bits[4];  // the lane's eight channels 8 lg .. 8 lg + 7 as they are stored
 #pragma unroll
                 for (int mb = 0; mb < 2; ++mb) {
                     float v[4];
@@ -751,25 +775,23 @@ __global__ __launch_bounds__(256, (convBlocksPerCu<IN, OUT, AIN>())) void conv3x
                                        : acc[mb][nb][r] + bv[mb][r];
                         if (kBf16 && relu) v[r] = gmax(v[r], 0.0f);
                     }
-                    const int co = mb * 16 + 4 * lg;
                     if constexpr (OUT == OUT_F32) {
                         static_assert(!kScaled, "FP32 activations are a BF16 (training) form");
                         if (x < W && y < H)
-                            *reinterpret_cast<float4*>(static_cast<float*>(out) + p * kC + co) =
+                            *reinterpret_cast<float4*>(static_cast<float*>(out) + p * kC + mb * 16 + 4 * lg) =
                                 make_float4(v[0], v[1], v[2], v[3]);
                     } else if constexpr (AOUT == ACT_F8) {
-                        const uint32_t q = packF8x4(v[0], v[1], v[2], v[3]);
-                        if (x < W && y < H) *reinterpret_cast<uint32_t*>(static_cast<uint8_t*>(out) + p * kC + co) = q;
+                        bits[mb] = packF8x4(v[0], v[1], v[2], v[3]);
                         if constexpr (OUT == OUT_BF16_POOL) {  // keep the stored values for the pooling
                             float d[4];
-                            unpackF8x4(q, d);
+                            unpackF8x4(bits[mb], d);
 #pragma unroll
                             for (int r = 0; r < 4; ++r) acc[mb][nb][r] = d[r];
                         }
                     } else {
                         const uint32_t b01 = f2bf2(v[0], v[1]), b23 = f2bf2(v[2], v[3]);
-                        if (x < W && y < H)
-                            *reinterpret_cast<uint2*>(static_cast<uint16_t*>(out) + p * kC + co) = make_uint2(b01, b23);
+                        bits[2 * mb] = b01;
+                        bits[2 * mb + 1] = b23;
                         if constexpr (OUT == OUT_BF16_POOL) {  // keep the stored values for the pooling
                             acc[mb][nb][0] = bf2f((uint16_t)(b01 & 0xffffu));
                             acc[mb][nb][1] = bf2f((uint16_t)(b01 >> 16));
@@ -778,43 +800,51 @@ __global__ __launch_bounds__(256, (convBlocksPerCu<IN, OUT, AIN>())) void conv3x
                         }
                     }
                 }
+                if (kBf16 && x < W && y < H) storeChannels<AOUT>(out, p, lg, bits);
             }
             if constexpr (OUT == OUT_BF16_POOL) {
                 // rows 4 wave + {0, 1} and {2, 3} pool into two coarse rows; the even lane
                 // of each column pair sums its children in poolKernel's order
                 const int cw = (W + 1) / 2;
                 const bool xIn = x < W, x1In = x + 1 < W, even = (l16 & 1) == 0;
+                const bool whole = (tx + 1) * kTS <= W && (ty + 1) * kTS <= H;  // no pixel is cut off
 #pragma unroll
                 for (int pr = 0; pr < 2; ++pr) {
                     const int y0 = ty * kTS + wave * 4 + 2 * pr;
                     const bool y1In = y0 + 1 < H;
                     const int n = (1 + (x1In ? 1 : 0)) * (1 + (y1In ? 1 : 0));
                     const float inv = n == 4 ? 0.25f : (n == 2 ? 0.5f : 1.0f);  // 1 / n, exact
+                    uint32_t bits[4];
 #pragma unroll
                     for (int mb = 0; mb < 2; ++mb) {
                         float m[4];
 #pragma unroll
                         for (int r = 0; r < 4; ++r) {
                             const float a00 = acc[mb][2 * pr][r], a10 = acc[mb][2 * pr + 1][r];
-                            const float a01 = __shfl_xor(a00, 1), a11 = __shfl_xor(a10, 1);
+                            const float a01 = columnNeighbour(a00), a11 = columnNeighbour(a10);
                             float sum = 0.0f;
                             sum += a00;
-                            if (x1In) sum += a01;
-                            if (y1In) {
-                                sum += a10;
-                                if (x1In) sum += a11;
+                            if (whole) {
+                                sum = ((sum + a01) + a10) + a11;
+                                m[r] = sum * 0.25f;
+                            } else {
+                                if (x1In) sum += a01;
+                                if (y1In) {
+                                    sum += a10;
+                                    if (x1In) sum += a11;
+                                }
+                                m[r] = sum * inv;
                             }
-                            m[r] = sum * inv;
                         }
-                        const size_t q = ((size_t)(y0 / 2) * cw + x / 2) * kC + mb * 16 + 4 * lg;
                         if constexpr (AOUT == ACT_F8) {
-                            const uint32_t o = packF8x4(m[0], m[1], m[2], m[3]);
-                            if (even && xIn && y0 < H) *reinterpret_cast<uint32_t*>(reinterpret_cast<uint8_t*>(src.pooled) + q) = o;
+                            bits[mb] = packF8x4(m[0], m[1], m[2], m[3]);
                         } else {
-                            const uint32_t o01 = f2bf2(m[0], m[1]), o23 = f2bf2(m[2], m[3]);
-                            if (even && xIn && y0 < H) *reinterpret_cast<uint2*>(src.pooled + q) = make_uint2(o01, o23);
+                            bits[2 * mb] = f2bf2(m[0], m[1]);
+                            bits[2 * mb + 1] = f2bf2(m[2], m[3]);
                         }
                     }
+                    if (even && xIn && y0 < H)
+                        storeChannels<AOUT>(src.pooled, (size_t)(y0 / 2) * cw + x / 2, lg, bits);
                 }
             }
         }
