@@ -90,3 +90,29 @@ def test_converged_drops_only_rejected(radius, accumulate_fp64):
     assert orc.rel_l2(res.cpu().numpy(), orr) <= REL_L2
     assert float(np.abs(res[..., 3].cpu().numpy().astype(np.float64) - orr[..., 3]).max()) < 1e-3
     assert orc.rel_l2(col.cpu().numpy(), oc) <= REL_L2
+
+
+@pytest.fixture(scope="module")
+def city():
+    return Case(small(sc.CITY_1080P, name="city-200x120-1500vpl", width=200, height=120, num_vpls=1500, cube_res=8,
+                      csm_res=256))
+
+
+@pytest.mark.parametrize("radius", [None, -40.0, 0.0, 60.0, 1.0e6, float("nan")])
+@pytest.mark.parametrize("ts,K", [(8, 64), (16, 64), (16, 12), (32, 64)])
+def test_tile_lists_by_rank(city, ts, K, radius):
+    """Tile lists formed by counting smaller keys, against the oracle bit for bit: as generated, radii that
+    leave more candidates than there are keys, none, or negative ratios (the insertions run instead)."""
+    torch = require_gpu()
+    gi = GiPass(city.w.width, city.w.height, ts, K)
+    gi.set_frame(city.dev.frame)
+    gi.set_csm(city.dev.csm_struct())
+    upd, vis, _ = city.oracle_cull()
+    if radius is not None:
+        upd = upd.copy()
+        upd[:, 12] = radius
+    _, want = orc.cull_tiles(city.host.frame, city.hg, ts, K, upd, vis)
+    tiles = torch.full((gi.num_tiles, 1 + K), -5, dtype=torch.int32, device="cuda")
+    gi.cull_tiles(city.dev.gbuffer(), torch.from_numpy(upd).cuda(), torch.from_numpy(vis).cuda(), tiles)
+    torch.cuda.synchronize()
+    assert_tiles_equal(tiles.cpu().numpy(), want)
