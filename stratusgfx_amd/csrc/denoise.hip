@@ -258,11 +258,30 @@ __global__ __launch_bounds__(256) void denoiseFilterKernel(GbufArgs g, const flo
     filterRegion<S>(g, resIn, normals, resOut, (int)xcdSwizzle(blockIdx.x, gridDim.x));
 }
 
+// One pixel per thread, for images too small to fill the card with columns (usesColumns).
+__global__ __launch_bounds__(256) void denoiseFilterPixelKernel(GbufArgs g, int stride,
+                                                                const float4* __restrict__ resIn,
+                                                                const float4* __restrict__ normals,
+                                                                float4* __restrict__ resOut) {
+    int x, y;
+    blockPixel(g.W, g.H, x, y);
+    filterBody(g, stride, resIn, normals, resOut, x, y);
+}
+
 __global__ __launch_bounds__(256) void denoiseFilterListKernel(GbufArgs g, int stride, const float4* __restrict__ resIn,
                                                                const float4* __restrict__ normals,
                                                                float4* __restrict__ resOut,
                                                                const int32_t* __restrict__ list) {
     forListedTiles(list, g.W, [&](int x, int y) { filterBody(g, stride, resIn, normals, resOut, x, y); });
+}
+
+__global__ __launch_bounds__(256) void denoiseFilterViewsPixelKernel(const sgi_batch::ViewDesc* __restrict__ views,
+                                                                     int numViews, int total, int pass) {
+    int x, y;
+    const sgi_batch::ViewDesc& d = viewBlock(views, numViews, total, x, y);
+    const float4* in = pass == 2 ? d.resB : d.resA;
+    float4* out = pass == 1 ? d.resB : (pass == 2 ? d.resA : (float4*)d.reservoirOut);
+    filterBody(d.g, 1 << pass, in, d.normals, out, x, y);
 }
 
 // pass 1: resA -> resB, pass 2: resB -> resA, pass 3: resA -> reservoirOut; region blocks in view order
@@ -472,6 +491,13 @@ hipError_t taa(const float* screen, const float* prev, const float* velocity, in
     return hipGetLastError();
 }
 
+// Whether the a-trous passes run over columns of four pixels, from the number of 64 x 4 pixel blocks: with
+// one wave or less per SIMD a column's four-fold chain decides, with more its fewer loads do.
+// The whole denoiser by pixels / columns: 320x180 18 / 30 us, 560x315 (711 blocks) 33.3 / 35.1, 640x360
+// (900) 40.3 / 37.2, 960x540 68 / 56.
+constexpr int kColumnBlocks = 800;
+static bool usesColumns(int blocks) { return blocks >= kColumnBlocks; }
+
 hipError_t denoiseSpatial(const GbufArgs& cur, const FrameArgs& fr, const int32_t* visible, const float* reservoir,
                           float* reservoirOut, const DenoiseBuffers& ws, const int32_t* tiles, bool mergeOnly,
                           hipStream_t s) {
@@ -490,6 +516,14 @@ hipError_t denoiseSpatial(const GbufArgs& cur, const FrameArgs& fr, const int32_
         for (int pass = 0; pass < 3 && e == hipSuccess; ++pass) {
             hipLaunchKernelGGL(denoiseFilterListKernel, lgrid, block, 0, s, cur, 2 << pass, in[pass], ws.normals,
                                out[pass], tiles);
+            e = hipGetLastError();
+        }
+        return e;
+    }
+    if (!usesColumns((int)grid.x)) {
+        for (int pass = 0; pass < 3 && e == hipSuccess; ++pass) {
+            hipLaunchKernelGGL(denoiseFilterPixelKernel, grid, block, 0, s, cur, 2 << pass, in[pass], ws.normals,
+                               out[pass]);
             e = hipGetLastError();
         }
         return e;
@@ -535,9 +569,15 @@ hipError_t denoiseViews(const sgi_batch::ViewDesc* views, int numViews, int tota
     hipLaunchKernelGGL(denoiseMergeViewsKernel, dim3(totalBlocks), dim3(256), 0, s, views, numViews, totalBlocks);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(denoiseFilterViewsKernel<1>, dim3(totalFilter), dim3(256), 0, s, views, numViews);
-    hipLaunchKernelGGL(denoiseFilterViewsKernel<2>, dim3(totalFilter), dim3(256), 0, s, views, numViews);
-    hipLaunchKernelGGL(denoiseFilterViewsKernel<3>, dim3(totalFilter), dim3(256), 0, s, views, numViews);
+    if (usesColumns(totalBlocks)) {
+        hipLaunchKernelGGL(denoiseFilterViewsKernel<1>, dim3(totalFilter), dim3(256), 0, s, views, numViews);
+        hipLaunchKernelGGL(denoiseFilterViewsKernel<2>, dim3(totalFilter), dim3(256), 0, s, views, numViews);
+        hipLaunchKernelGGL(denoiseFilterViewsKernel<3>, dim3(totalFilter), dim3(256), 0, s, views, numViews);
+    } else {
+        for (int pass = 1; pass <= 3; ++pass)
+            hipLaunchKernelGGL(denoiseFilterViewsPixelKernel, dim3(totalBlocks), dim3(256), 0, s, views, numViews,
+                               totalBlocks, pass);
+    }
     e = hipGetLastError();
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(denoiseTemporalViewsKernel, dim3(totalBlocks), dim3(256), 0, s, views, numViews, totalBlocks);

@@ -1,4 +1,5 @@
-"""The a-trous filter at the edges of its regions: a thread filters four pixels of a column that lie a
+"""The a-trous filter at the edges of its regions, in both forms: one pixel per thread below 800 blocks of
+64 x 4 pixels, and from there on (517 x 375 here) a thread filters four pixels of a column that lie a
 lattice step (2, 4, 8) apart, regions are 64 x 32 pixels, and pixels past the frame's last row or column
 have to stay unwritten."""
 import numpy as np
@@ -14,7 +15,7 @@ pytestmark = pytest.mark.gpu
 REL_L2 = 1e-4  # FP32 images, the bound of every parity test
 
 
-@pytest.mark.parametrize("W,H", [(1, 1), (3, 33), (64, 32), (65, 31), (63, 40), (130, 70)])
+@pytest.mark.parametrize("W,H", [(1, 1), (3, 33), (64, 32), (65, 31), (63, 40), (130, 70), (517, 375), (64, 3203), (2049, 97)])
 def test_denoise_matches_oracle(W, H):
     torch = require_gpu()
     case = Case(small(sc.CORNELL_640x360, name=f"cornell-{W}x{H}-12vpl", width=W, height=H, num_vpls=12,
