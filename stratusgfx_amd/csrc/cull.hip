@@ -110,6 +110,42 @@ __global__ __launch_bounds__(kCullThreads) void cullCompactKernel(const sgi_vpl*
     cullCompactBody(in, n, flags, out, visible, waveCount);
 }
 
+// The same compaction over many blocks of kSplitThreads items, each counting the flags before its own (a
+// few KB from L2) instead of waiting for an earlier block.  The copies of 64 B records are then spread
+// over the CUs: 4096 VPLs 16 -> 4.8 us.
+constexpr int kSplitThreads = 256, kSplitMin = 256;
+__global__ __launch_bounds__(kSplitThreads) void cullCompactSplitKernel(const sgi_vpl* __restrict__ in, int n,
+                                                                        const uint8_t* __restrict__ flags,
+                                                                        sgi_vpl* __restrict__ out,
+                                                                        int32_t* __restrict__ visible) {
+    __shared__ int before[kSplitThreads / 64], within[kSplitThreads / 64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int first = (int)blockIdx.x * kSplitThreads, i = first + (int)threadIdx.x;
+    int earlier = 0;
+    for (int j = 4 * (int)threadIdx.x; j < first; j += 4 * kSplitThreads)  // flags are 0 or 1, four to a word
+        earlier += __popc(*reinterpret_cast<const uint32_t*>(flags + j));
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) earlier += __shfl_xor(earlier, o, 64);
+    const bool f = i < n && flags[i] != 0;
+    const uint64_t m = __ballot(f);
+    if (lane == 0) {
+        before[wave] = earlier;
+        within[wave] = __popcll(m);
+    }
+    __syncthreads();
+    int pos = __popcll(m & ((1ull << lane) - 1ull)), total = 0;
+#pragma unroll
+    for (int w = 0; w < kSplitThreads / 64; ++w) {
+        pos += before[w] + (w < wave ? within[w] : 0);
+        total += before[w] + within[w];
+    }
+    if (f && pos < SGI_MAX_TOTAL_VPLS_PER_FRAME) {
+        out[pos] = in[i];
+        visible[1 + pos] = i;
+    }
+    if (threadIdx.x == 0 && blockIdx.x == gridDim.x - 1) visible[0] = min(total, SGI_MAX_TOTAL_VPLS_PER_FRAME);
+}
+
 // Batched: one block per view.
 __global__ __launch_bounds__(kCullThreads) void cullCompactViewsKernel(const sgi_batch::ViewDesc* __restrict__ views,
                                                                        const sgi_vpl* __restrict__ in, int n) {
@@ -473,7 +509,14 @@ hipError_t cullGlobal(const CsmArgs& csm, const FrameArgs& fr, const sgi_vpl* in
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
     }
-    hipLaunchKernelGGL(cullCompactKernel, dim3(1), dim3(kCullThreads), 0, s, in, n, flags, out, visible);
+    // one block where it takes its items in one round, where out lies over in (it reads before it writes) or
+    // the flags cannot be read by words: 1024 VPLs 5.5 us in one block, 4.7 split
+    const bool apart = out + n <= in || in + n <= out;
+    if (n > kSplitMin && apart && (uintptr_t)flags % 4 == 0)
+        hipLaunchKernelGGL(cullCompactSplitKernel, dim3((n + kSplitThreads - 1) / kSplitThreads), dim3(kSplitThreads),
+                           0, s, in, n, flags, out, visible);
+    else
+        hipLaunchKernelGGL(cullCompactKernel, dim3(1), dim3(kCullThreads), 0, s, in, n, flags, out, visible);
     return hipGetLastError();
 }
 

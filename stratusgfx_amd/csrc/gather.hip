@@ -765,9 +765,8 @@ __global__ __launch_bounds__(256) void gatherSamplesKernel(GbufArgs g, FrameArgs
 // What bounds it is the vector L1: a lane's random line costs an access for each load instruction, and
 // it was busy 84 % of the time (the vector ALU 54 %).  A record is read by four lanes in one access
 // and handed over through LDS instead of by one lane in four; pixels' rows are cut to 64 B so that four
-// blocks still
-// fit a CU (38.9 KB each; at three, 5 % slower where the records hit L1 anyway).  1080p, 32 draws, 4096
-// lights: 527 -> 492 us.
+// blocks still fit a CU (38.9 KB each; at three, 5 % slower where the records hit L1 anyway).  1080p,
+// 32 draws, 4096 lights: 527 -> 492 us; 1279x717, 2048 lights: the gather alone 157 -> 146.
 constexpr int kDrawBatch = 8;
 
 __device__ __forceinline__ void waveSync() {
