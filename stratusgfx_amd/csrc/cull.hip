@@ -207,15 +207,17 @@ __global__ void gatherEntriesViewsKernel(const sgi_batch::ViewDesc* __restrict__
 // A tile-culling block's LDS: the per-pixel components that stage 1 sums (six planes at once, three at a
 // time for 32x32 tiles), each plane 4 floats longer than the tile so that the summing lanes read different
 // banks; then, in the same words, stage 2's histogram (256 counters), compacted slot list (kListCap) and
-// ratio codes (a byte per VPL), and over the codes the candidates' keys.  6.2 KB for 8x8 and 16x16 tiles:
-// 26 one-wave blocks per CU.
-constexpr int kListCap = 1024, kKeyCap = 256;
+// ratio codes (a byte per VPL), and over the codes the candidates' keys.  6.5 KB for 8x8 and 16x16 tiles:
+// 24 one-wave blocks per CU.  (Room for 3168 codes in 6.2 KB is 1-5 % faster up to 2048 VPLs, and 4096 then
+// scan twice: 163 us and not 109.)
+constexpr int kListCap = 512, kKeyCap = 256;
 template <int TS>
 struct CullLds {
     static constexpr int kStride = TS * TS + 4;
     static constexpr int kPlanes = TS <= 16 ? 6 : 3;
     static constexpr int kCodesAt = 256 + kListCap / 2;  // in words
-    static constexpr int kWords = kPlanes * kStride > 6 * 260 ? kPlanes * kStride : 6 * 260;
+    static constexpr int kStage2 = kCodesAt + SGI_MAX_TOTAL_VPLS_PER_FRAME / 4;
+    static constexpr int kWords = kPlanes * kStride > kStage2 ? kPlanes * kStride : kStage2;
     static constexpr int kCodeCap = (kWords - kCodesAt) * 4;
     static_assert(kCodesAt % 2 == 0 && kKeyCap * 8 <= kCodeCap, "the keys lie over the codes");
 };
@@ -309,7 +311,7 @@ __device__ __forceinline__ void cullTileBody(const GbufArgs& g, const FrameArgs&
     // the sums are formed).
     uint32_t* hist = reinterpret_cast<uint32_t*>(comp);
     uint8_t* codes = reinterpret_cast<uint8_t*>(hist + Lds::kCodesAt);
-    const bool haveCodes = numVisible <= Lds::kCodeCap;
+    const bool haveCodes = numVisible <= Lds::kCodeCap;  // unless the caller counts more than a frame holds
     for (int i = lane; i < 256; i += 64) hist[i] = 0u;
     __syncthreads();
     for (int b = 0; b < numVisible; b += 64) {
@@ -379,7 +381,7 @@ __device__ __forceinline__ void cullTileBody(const GbufArgs& g, const FrameArgs&
     // order): the list wanted is the K smallest keys in order, and a candidate's place in it is the
     // number of smaller keys.  Counting them takes two instructions a pair of 64 candidates and key;
     // inserting one by one took some twenty per candidate.  With the sums side by side and the codes: 1080p,
-    // 1024 VPLs 66 -> 45 us; eight 720p views, 512 VPLs 83 -> 57; 640x360, 64 VPLs 16 -> 10.
+    // 1024 VPLs 64 -> 45 us, 4096 172 -> 109; eight 720p views, 512 VPLs 83 -> 57; 640x360, 64 VPLs 16 -> 10.
     uint64_t* keys = reinterpret_cast<uint64_t*>(codes);
     if (useList) {
         int m = 0;
