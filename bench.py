@@ -180,9 +180,9 @@ def culling_roofline(per_plain, W, H, tiles, K, visible, num_vpls):
         out[name] = {"bound": "hbm", "achieved": round(ach, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(ach / HBM_PEAK_GBS, 4), "traffic": traffic, "algorithmic_bytes": int(alg),
                      "avg_launch_ms": round(ms, 4)}
-    out["cull_global"]["kernels"] = "cullVisibilityKernel + cullCompactKernel"
+    out["cull_global"]["kernels"] = "cullVisibilityKernel + cullCompactSplitKernel"
     out["cull_tiles"]["kernels"] = "cullTilesKernel<16>"
-    out["note"] = ("neither stage is HBM-bound: the global cull is two launches of 64 and 16 waves over 4096 VPLs "
+    out["note"] = ("neither stage is HBM-bound: the global cull is two launches of 64 and 64 waves over 4096 VPLs "
                    "(latency), the tile cull one wave per tile against every visible VPL (VALU for the estimated "
                    "ratios and the exact ones below the histogram bound, and the serial stage-1 sums; "
                    "profiles/valu_counters_gather_samples_city1080p.md)")

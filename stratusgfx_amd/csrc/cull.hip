@@ -1,6 +1,6 @@
 // VPL culling kernels.
 //
-// cullVisibilityKernel + cullCompactKernel — viscull_vpls.cs:47-120: per VPL,
+// cullVisibilityKernel + cullCompactSplitKernel (cullCompactKernel for a few) — viscull_vpls.cs:47-120: per VPL,
 // the sun-visibility test through the cascades, then a stable compaction (wave
 // ballot + block prefix) of the visible records in ascending input order.
 //
@@ -9,10 +9,10 @@
 // tile's pixels in parallel into LDS and then sums each of the six components
 // serially in row-major local order, which is the reference's summation order
 // (thread 0's loop), so the tile mean is bit-identical.  Stage 2 evaluates 64
-// VPLs per step across the lanes and keeps the sorted top-K list in lane
-// registers (lane k holds entry k); candidates below the current K-th ratio
-// are inserted one at a time in slot order with a ballot for the position and
-// a lane shift, which reproduces the reference's strict-< insertion sort.
+// VPLs per step across the lanes; the K-th ratio is bounded by a histogram, and
+// each candidate below the bound finds its place in the list by counting the
+// smaller keys (ratio, slot order), which is the reference's stable strict-<
+// insertion sort.
 //
 // colorVplsKernel — vpl_light_color.cs:41-76: one thread per visible slot
 // reads the diffuse and distance texels in direction -sun and writes the
@@ -300,7 +300,7 @@ __device__ __forceinline__ void cullTileBody(const GbufArgs& g, const FrameArgs&
 
     const int numVisible = visible[0];
     // Stage 2a: an upper bound of the K-th smallest candidate ratio, so that stage 2 inserts
-    // little beyond the final list (the insertions, not the ratios, dominate its cost). A
+    // little beyond the final list. A
     // 256-bucket histogram over [0, 1) of estimated ratios (hardware sqrt and reciprocal: within
     // 2^-21 relative of the correctly rounded ratio) counts only VPLs that are certainly
     // candidates (the exact side test, estimate <= 1 - 2^-18). If K of them fall in buckets up to
