@@ -253,8 +253,9 @@ int sgi_gbuffer_unpack(sgi_ctx* ctx, const sgi_gbuffer_packed* g, float* normal,
     return e == hipSuccess ? SGI_OK : hipFail(e, "sgi_gbuffer_unpack");
 }
 
-int sgi_cull_global(sgi_ctx* ctx, const sgi_vpl* vplData, int32_t n, sgi_vpl* vplUpdatedData, int32_t* visibleIndices,
-                    void* stream) {
+// sgi_cull_global, with the visible slots' atlas entries (all, entries) or NULL
+static int cullGlobal(sgi_ctx* ctx, const sgi_vpl* vplData, int32_t n, sgi_vpl* vplUpdatedData,
+                      int32_t* visibleIndices, const sgi_atlas_entry* all, sgi_atlas_entry* entries, void* stream) {
     if (!ctx) return fail(SGI_E_INVALID, "sgi_cull_global: NULL context");
     if (!ctx->hasFrame || !ctx->hasCsm) return fail(SGI_E_STATE, "sgi_cull_global: sgi_set_frame and sgi_set_csm first");
     if (n < 0 || n > SGI_MAX_TOTAL_VPLS_BEFORE_CULLING)
@@ -264,8 +265,14 @@ int sgi_cull_global(sgi_ctx* ctx, const sgi_vpl* vplData, int32_t n, sgi_vpl* vp
     if (n > 0 && (!aligned16(vplData) || !aligned16(vplUpdatedData)))
         return fail(SGI_E_INVALID, "sgi_cull_global: VPL records must be 16-byte aligned");
     const hipError_t e = sgi_launch::cullGlobal(ctx->csmArgs, ctx->frameArgs, vplData, n, vplUpdatedData,
-                                                visibleIndices, ctx->visFlags, (hipStream_t)stream);
+                                                visibleIndices, ctx->visFlags, all, entries,
+                                                (hipStream_t)stream);
     return e == hipSuccess ? SGI_OK : hipFail(e, "sgi_cull_global");
+}
+
+int sgi_cull_global(sgi_ctx* ctx, const sgi_vpl* vplData, int32_t n, sgi_vpl* vplUpdatedData, int32_t* visibleIndices,
+                    void* stream) {
+    return cullGlobal(ctx, vplData, n, vplUpdatedData, visibleIndices, nullptr, nullptr, stream);
 }
 
 int sgi_visible_atlas_entries(sgi_ctx* ctx, const sgi_atlas_entry* shadowIndices, const int32_t* visibleIndices,
@@ -459,12 +466,16 @@ int sgi_render_frame(sgi_ctx* ctx, const sgi_frame_io* io, void* stream) {
         return fail(SGI_E_INVALID, "sgi_render_frame: NULL atlas entry buffer");
     if (io->useTiles && !io->tiles) return fail(SGI_E_INVALID, "sgi_render_frame: tile lists requested, tiles NULL");
     // UpdatePointLights_ -> PerformVirtualPointLightCullingStage1_
-    int r = sgi_cull_global(ctx, io->vplData, io->numVpls, io->vplUpdatedData, io->visibleIndices, stream);
-    if (r != SGI_OK) return r;
-    // PerformVirtualPointLightCullingStage2_: atlas entries of the visible slots
+    // with PerformVirtualPointLightCullingStage2_'s atlas entries of the visible slots, unless they
+    // replace the entries they are taken from
     const int maxCount = io->numVpls < SGI_MAX_TOTAL_VPLS_PER_FRAME ? io->numVpls : SGI_MAX_TOTAL_VPLS_PER_FRAME;
-    if ((r = sgi_visible_atlas_entries(ctx, io->shadowIndices, io->visibleIndices, maxCount,
-                                       io->visibleShadowIndices, stream)) != SGI_OK)
+    const bool apart = io->visibleShadowIndices + maxCount <= io->shadowIndices ||
+                       io->shadowIndices + io->numVpls <= io->visibleShadowIndices;
+    int r = cullGlobal(ctx, io->vplData, io->numVpls, io->vplUpdatedData, io->visibleIndices,
+                       apart ? io->shadowIndices : nullptr, io->visibleShadowIndices, stream);
+    if (r != SGI_OK) return r;
+    if (!apart && (r = sgi_visible_atlas_entries(ctx, io->shadowIndices, io->visibleIndices, maxCount,
+                                                 io->visibleShadowIndices, stream)) != SGI_OK)
         return r;
     // PerformVirtualPointLightCullingStage2_: the vplColoring dispatch (vpl_light_color.cs)
     if (io->diffuseCubes &&

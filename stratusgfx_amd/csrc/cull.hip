@@ -53,6 +53,8 @@ __global__ __launch_bounds__(64) void cullVisibilityViewsKernel(const sgi_batch:
     cullVisibilityBody(d.csm, ld3(d.fr.sunDir), in, n, d.visFlags, (blockIdx.x % bpv) * 64 + threadIdx.x);
 }
 
+// With `all` given, the visible VPLs' atlas entries are written with their records (a frame's and a
+// batch's next launch was that copy: 2 us of a 640x360 frame).
 // Stable compaction of the flags: wave ballots and a block prefix, in input
 // order. The block takes kCompactRounds chunks of kCullThreads items at a
 // time: the chunks' flags are loaded together before the one barrier, then
@@ -62,6 +64,8 @@ __global__ __launch_bounds__(64) void cullVisibilityViewsKernel(const sgi_batch:
 constexpr int kCompactRounds = 4;
 __device__ __forceinline__ void cullCompactBody(const sgi_vpl* __restrict__ in, int n, const uint8_t* __restrict__ flags,
                                                 sgi_vpl* __restrict__ out, int32_t* __restrict__ visible,
+                                                const sgi_atlas_entry* __restrict__ all,
+                                                sgi_atlas_entry* __restrict__ entries,
                                                 int (*waveCount)[kCullThreads / 64]) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const uint64_t below = lane == 0 ? 0ull : (~0ull >> (64 - lane));
@@ -94,6 +98,7 @@ __device__ __forceinline__ void cullCompactBody(const sgi_vpl* __restrict__ in, 
                 const int i = c0 + k * kCullThreads + (int)threadIdx.x;
                 out[pos] = in[i];
                 visible[1 + pos] = i;
+                if (all) entries[pos] = all[i];
             }
             running += total;
         }
@@ -105,9 +110,11 @@ __device__ __forceinline__ void cullCompactBody(const sgi_vpl* __restrict__ in, 
 __global__ __launch_bounds__(kCullThreads) void cullCompactKernel(const sgi_vpl* __restrict__ in, int n,
                                                                   const uint8_t* __restrict__ flags,
                                                                   sgi_vpl* __restrict__ out,
-                                                                  int32_t* __restrict__ visible) {
+                                                                  int32_t* __restrict__ visible,
+                                                                  const sgi_atlas_entry* __restrict__ all,
+                                                                  sgi_atlas_entry* __restrict__ entries) {
     __shared__ int waveCount[kCompactRounds][kCullThreads / 64];
-    cullCompactBody(in, n, flags, out, visible, waveCount);
+    cullCompactBody(in, n, flags, out, visible, all, entries, waveCount);
 }
 
 // The same compaction over many blocks of kSplitThreads items, each counting the flags before its own (a
@@ -117,7 +124,9 @@ constexpr int kSplitThreads = 256, kSplitMin = 256;
 __global__ __launch_bounds__(kSplitThreads) void cullCompactSplitKernel(const sgi_vpl* __restrict__ in, int n,
                                                                         const uint8_t* __restrict__ flags,
                                                                         sgi_vpl* __restrict__ out,
-                                                                        int32_t* __restrict__ visible) {
+                                                                        int32_t* __restrict__ visible,
+                                                                        const sgi_atlas_entry* __restrict__ all,
+                                                                        sgi_atlas_entry* __restrict__ entries) {
     __shared__ int before[kSplitThreads / 64], within[kSplitThreads / 64];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int first = (int)blockIdx.x * kSplitThreads, i = first + (int)threadIdx.x;
@@ -142,16 +151,18 @@ __global__ __launch_bounds__(kSplitThreads) void cullCompactSplitKernel(const sg
     if (f && pos < SGI_MAX_TOTAL_VPLS_PER_FRAME) {
         out[pos] = in[i];
         visible[1 + pos] = i;
+        if (all) entries[pos] = all[i];
     }
     if (threadIdx.x == 0 && blockIdx.x == gridDim.x - 1) visible[0] = min(total, SGI_MAX_TOTAL_VPLS_PER_FRAME);
 }
 
 // Batched: one block per view.
 __global__ __launch_bounds__(kCullThreads) void cullCompactViewsKernel(const sgi_batch::ViewDesc* __restrict__ views,
-                                                                       const sgi_vpl* __restrict__ in, int n) {
+                                                                       const sgi_vpl* __restrict__ in, int n,
+                                                                       const sgi_atlas_entry* __restrict__ all) {
     __shared__ int waveCount[kCompactRounds][kCullThreads / 64];
     const sgi_batch::ViewDesc& d = views[blockIdx.x];
-    cullCompactBody(in, n, d.visFlags, d.vplUpdated, d.visible, waveCount);
+    cullCompactBody(in, n, d.visFlags, d.vplUpdated, d.visible, all, d.entries, waveCount);
 }
 
 __global__ void gatherEntriesKernel(const sgi_atlas_entry* __restrict__ all, const int32_t* __restrict__ visible,
@@ -193,15 +204,6 @@ __global__ __launch_bounds__(256) void colorVplsKernel(CubeArgs diffuse, CubeArg
     }
     v.color[3] = 1.0f;
     v.specularPosition[3] = 1.0f;
-}
-
-// Batched: blocks [v * bpv, (v + 1) * bpv) gather view v's visible slots.
-__global__ void gatherEntriesViewsKernel(const sgi_batch::ViewDesc* __restrict__ views,
-                                         const sgi_atlas_entry* __restrict__ all, int maxCount, int bpv) {
-    const sgi_batch::ViewDesc& d = views[blockIdx.x / bpv];
-    const int s = (blockIdx.x % bpv) * blockDim.x + threadIdx.x;
-    const int count = d.visible[0];
-    if (s < count && s < maxCount) d.entries[s] = all[d.visible[1 + s]];
 }
 
 // A tile-culling block's LDS: the per-pixel components that stage 1 sums (six planes at once, three at a
@@ -505,7 +507,8 @@ __global__ __launch_bounds__(64) void cullTilesViewsKernel(const sgi_batch::View
 namespace sgi_launch {
 
 hipError_t cullGlobal(const CsmArgs& csm, const FrameArgs& fr, const sgi_vpl* in, int n, sgi_vpl* out,
-                      int32_t* visible, uint8_t* flags, hipStream_t s) {
+                      int32_t* visible, uint8_t* flags, const sgi_atlas_entry* all, sgi_atlas_entry* entries,
+                      hipStream_t s) {
     if (n > 0) {
         hipLaunchKernelGGL(cullVisibilityKernel, dim3((n + 63) / 64), dim3(64), 0, s, csm, ld3(fr.sunDir), in, n, flags);
         const hipError_t e = hipGetLastError();
@@ -516,9 +519,10 @@ hipError_t cullGlobal(const CsmArgs& csm, const FrameArgs& fr, const sgi_vpl* in
     const bool apart = out + n <= in || in + n <= out;
     if (n > kSplitMin && apart && (uintptr_t)flags % 4 == 0)
         hipLaunchKernelGGL(cullCompactSplitKernel, dim3((n + kSplitThreads - 1) / kSplitThreads), dim3(kSplitThreads),
-                           0, s, in, n, flags, out, visible);
+                           0, s, in, n, flags, out, visible, all, entries);
     else
-        hipLaunchKernelGGL(cullCompactKernel, dim3(1), dim3(kCullThreads), 0, s, in, n, flags, out, visible);
+        hipLaunchKernelGGL(cullCompactKernel, dim3(1), dim3(kCullThreads), 0, s, in, n, flags, out, visible, all,
+                           entries);
     return hipGetLastError();
 }
 
@@ -552,14 +556,15 @@ hipError_t cullTiles(const GbufArgs& g, const FrameArgs& fr, int tileSize, int t
     return hipGetLastError();
 }
 
-hipError_t cullGlobalViews(const sgi_batch::ViewDesc* views, int numViews, const sgi_vpl* in, int n, hipStream_t s) {
+hipError_t cullGlobalViews(const sgi_batch::ViewDesc* views, int numViews, const sgi_vpl* in, int n,
+                           const sgi_atlas_entry* all, hipStream_t s) {
     if (n > 0) {
         const int bpv = (n + 63) / 64;
         hipLaunchKernelGGL(cullVisibilityViewsKernel, dim3(numViews * bpv), dim3(64), 0, s, views, in, n, bpv);
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
     }
-    hipLaunchKernelGGL(cullCompactViewsKernel, dim3(numViews), dim3(kCullThreads), 0, s, views, in, n);
+    hipLaunchKernelGGL(cullCompactViewsKernel, dim3(numViews), dim3(kCullThreads), 0, s, views, in, n, all);
     return hipGetLastError();
 }
 
@@ -579,14 +584,6 @@ hipError_t colorVpls(const sgi_dev::CubeArgs& diffuse, const sgi_dev::CubeArgs& 
     else
         hipLaunchKernelGGL(colorVplsKernel<SGI_TEXEL_F32>, grid, dim3(256), 0, s, diffuse, dist, sun, col, mult,
                            visible, maxCount, entries, vpls);
-    return hipGetLastError();
-}
-
-hipError_t gatherVisibleEntriesViews(const sgi_batch::ViewDesc* views, int numViews, const sgi_atlas_entry* all,
-                                     int maxCount, hipStream_t s) {
-    if (maxCount <= 0) return hipSuccess;
-    const int bpv = (maxCount + 255) / 256;
-    hipLaunchKernelGGL(gatherEntriesViewsKernel, dim3(numViews * bpv), dim3(256), 0, s, views, all, maxCount, bpv);
     return hipGetLastError();
 }
 

@@ -11,7 +11,8 @@ namespace sgi_launch {
 
 // flags: device scratch of n bytes
 hipError_t cullGlobal(const sgi_dev::CsmArgs& csm, const sgi_dev::FrameArgs& fr, const sgi_vpl* in, int n,
-                      sgi_vpl* out, int32_t* visible, uint8_t* flags, hipStream_t s);
+                      sgi_vpl* out, int32_t* visible, uint8_t* flags, const sgi_atlas_entry* all,
+                      sgi_atlas_entry* entries, hipStream_t s);
 
 hipError_t gatherVisibleEntries(const sgi_atlas_entry* all, const int32_t* visible, int maxCount,
                                 sgi_atlas_entry* out, hipStream_t s);
@@ -89,9 +90,8 @@ hipError_t denoise(const sgi_dev::GbufArgs& cur, const sgi_dev::GbufArgs& prev, 
                    float* reservoirOut, float* historyOut, const DenoiseBuffers& ws, hipStream_t s);
 
 // Batched views (views: device array of ViewDesc, numbered in item order).
-hipError_t cullGlobalViews(const sgi_batch::ViewDesc* views, int numViews, const sgi_vpl* in, int n, hipStream_t s);
-hipError_t gatherVisibleEntriesViews(const sgi_batch::ViewDesc* views, int numViews, const sgi_atlas_entry* all,
-                                     int maxCount, hipStream_t s);
+hipError_t cullGlobalViews(const sgi_batch::ViewDesc* views, int numViews, const sgi_vpl* in, int n,
+                           const sgi_atlas_entry* all, hipStream_t s);
 hipError_t cullTilesViews(const sgi_batch::ViewDesc* views, int numViews, int totalTiles, int tileSize, int K,
                           hipStream_t s);
 hipError_t gatherViews(const sgi_batch::ViewDesc* views, int numViews, int totalTiles, int tileSize, int K,

@@ -19,7 +19,7 @@ void sgi_set_error(const std::string& msg);
 struct sgi_views {
     sgi_views_config cfg{};
     int device = 0;
-    int numViews = 0, totalTiles = 0, totalTiles16 = 0, totalBlocks = 0, totalFilter = 0, numVpls = 0, maxEntries = 0;
+    int numViews = 0, totalTiles = 0, totalTiles16 = 0, totalBlocks = 0, totalFilter = 0, numVpls = 0;
     const sgi_vpl* vpls = nullptr;
     const sgi_atlas_entry* shadowIndices = nullptr;
     sgi_dev::CubeArgs cubes{};
@@ -138,9 +138,7 @@ hipError_t sizeLearnedWorkspace(sgi_views* v) {
 
 hipError_t runStages(sgi_views* v, hipStream_t s) {
     const sgi_views_config& c = v->cfg;
-    hipError_t e = sgi_launch::cullGlobalViews(v->descs, v->numViews, v->vpls, v->numVpls, s);
-    if (e == hipSuccess)
-        e = sgi_launch::gatherVisibleEntriesViews(v->descs, v->numViews, v->shadowIndices, v->maxEntries, s);
+    hipError_t e = sgi_launch::cullGlobalViews(v->descs, v->numViews, v->vpls, v->numVpls, v->shadowIndices, s);
     if (e == hipSuccess) e = sgi_launch::directLightViews(v->descs, v->numViews, v->totalTiles16, s);
     if (v->samples > 0) {
         // the learned form: each view's sampled gather and network in turn (sizes differ per view)
@@ -319,7 +317,6 @@ int sgi_views_set(sgi_views* v, int32_t numViews, const sgi_view_io* io, const s
     v->totalBlocks = blocks;
     v->totalFilter = filter;
     v->numVpls = numVpls;
-    v->maxEntries = numVpls < cap ? numVpls : cap;
     v->vpls = vpls;
     v->shadowIndices = shadowIndices;
     v->cubes = ca;
