@@ -12,7 +12,7 @@
 //           denoiseTemporalKernel: the temporal blend with the reprojected
 //           history and the combine screen + albedo * gi.
 //
-// Blocks cover 64x4 pixels (the filter: eight rows spread over 64x32) and are numbered so that each XCD walks a
+// Blocks cover 64x4 pixels (the filter: eight waves over 64x16 or 64x32) and are numbered so that each XCD walks a
 // contiguous band of rows: the 5x5 taps at stride 8 reach 16 rows up and down,
 // and that window stays in the XCD's L2 instead of being fetched once per XCD.
 // The edge-stopping weights and the normalisation are continuous, so they use
@@ -186,41 +186,41 @@ __device__ __forceinline__ void filterBody(const GbufArgs& g, int stride, const 
     resOut[p] = make_float4(rf0 * inv, rf1 * inv, rf2 * inv, 1.0f);
 }
 
-// The same sums, in the same order, for four pixels of a column: rows y0, y0 + S, y0 + 2 S, y0 + 3 S of
-// column x lie on one lattice of the pass, so their taps are 5 x 8 texels and not 4 x 25, and y0 is the
-// same over the wave, so a tap's row costs no vector address.  One pixel per thread was bound by the
-// 800 B a pixel read through L1 (62 us a pass at 1080p, vector ALU 56 % busy); this form takes 40, 40 and
-// 50 us at strides 2, 4 and 8, against 12 us for the bytes and about 30 for the arithmetic.  The columns
-// of taps stay a loop: unrolled, their loads are hoisted and 350 registers leave one wave per SIMD.
-template <int S>
+// The same sums, in the same order, for R pixels of a column: rows y0, y0 + S, ... of column x lie on one
+// lattice of the pass, so for four of them the taps are 5 x 8 texels and not 4 x 25, and y0 is the same
+// over the wave, so a tap's row costs no vector address.  One pixel per thread was bound by the 800 B a
+// pixel read through L1 (62 us a pass at 1080p, vector ALU 56 % busy); four take 40, 40 and 50 us at
+// strides 2, 4 and 8, against 12 us for the bytes and about 30 for the arithmetic.  The columns of
+// taps stay a loop: unrolled, their loads are hoisted and 350 registers leave one wave per SIMD.
+template <int S, int R>
 __device__ __forceinline__ void filterColumn(const GbufArgs& g, const float4* __restrict__ resIn,
                                              const float4* __restrict__ normals, float4* __restrict__ resOut, int x,
                                              int y0) {
     const int W = g.W, H = g.H;
     const int xc = x < W ? x : W - 1;
-    const float4* nRow[8];
-    const float4* rRow[8];
+    const float4* nRow[R + 4];
+    const float4* rRow[R + 4];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
+    for (int j = 0; j < R + 4; ++j) {
         const size_t o = (size_t)clampx(y0 + (j - 2) * S, H) * W;
         nRow[j] = normals + o;
         rRow[j] = resIn + o;
     }
-    float4 cn[4];
+    float4 cn[R];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) cn[k] = nRow[k + 2][xc];
-    float rf[4][4] = {};
+    for (int k = 0; k < R; ++k) cn[k] = nRow[k + 2][xc];
+    float rf[R][4] = {};
 #pragma unroll 1
     for (int dx = -2; dx <= 2; ++dx) {
         const int tx = clampx(xc + dx * S, W);
-        float4 n[8], r[8];
+        float4 n[R + 4], r[R + 4];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
+        for (int j = 0; j < R + 4; ++j) {
             n[j] = nRow[j][tx];
             r[j] = rRow[j][tx];
         }
 #pragma unroll
-        for (int k = 0; k < 4; ++k)
+        for (int k = 0; k < R; ++k)
 #pragma unroll
             for (int dy = -2; dy <= 2; ++dy) {
                 const int j = k + 2 + dy;
@@ -232,7 +232,7 @@ __device__ __forceinline__ void filterColumn(const GbufArgs& g, const float4* __
             }
     }
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
+    for (int k = 0; k < R; ++k) {
         const int y = y0 + k * S;
         if (x >= W || y >= H) continue;
         const float inv = frcp(gmax(kEPS, rf[k][3]));
@@ -240,25 +240,25 @@ __device__ __forceinline__ void filterColumn(const GbufArgs& g, const float4* __
     }
 }
 
-// 64 x 32 pixel regions, eight waves each in two blocks: wave w of a region starts at row
-// (w / S) 4 S + w % S, so S waves cover 4 S rows.
-template <int S>
+// Regions of 64 x 8 R pixels, eight waves each in two blocks: wave w of a region starts at row
+// (w / S) R S + w % S, so S waves cover R S rows.
+template <int S, int R>
 __device__ __forceinline__ void filterRegion(const GbufArgs& g, const float4* __restrict__ resIn,
                                              const float4* __restrict__ normals, float4* __restrict__ resOut, int b) {
     const int regionsX = (g.W + 63) / 64, r = b >> 1;
     const int w = __builtin_amdgcn_readfirstlane((b & 1) * 4 + (int)(threadIdx.x >> 6));
-    const int y0 = (r / regionsX) * 32 + (w / S) * 4 * S + w % S;
-    filterColumn<S>(g, resIn, normals, resOut, (r % regionsX) * 64 + (int)(threadIdx.x & 63), y0);
+    const int y0 = (r / regionsX) * 8 * R + (w / S) * R * S + w % S;
+    filterColumn<S, R>(g, resIn, normals, resOut, (r % regionsX) * 64 + (int)(threadIdx.x & 63), y0);
 }
 
-template <int S>
+template <int S, int R>
 __global__ __launch_bounds__(256) void denoiseFilterKernel(GbufArgs g, const float4* __restrict__ resIn,
                                                            const float4* __restrict__ normals,
                                                            float4* __restrict__ resOut) {
-    filterRegion<S>(g, resIn, normals, resOut, (int)xcdSwizzle(blockIdx.x, gridDim.x));
+    filterRegion<S, R>(g, resIn, normals, resOut, (int)xcdSwizzle(blockIdx.x, gridDim.x));
 }
 
-// One pixel per thread, for images too small to fill the card with columns (usesColumns).
+// One pixel per thread, for images too small to fill the card with columns (sgi_batch::filterRows).
 __global__ __launch_bounds__(256) void denoiseFilterPixelKernel(GbufArgs g, int stride,
                                                                 const float4* __restrict__ resIn,
                                                                 const float4* __restrict__ normals,
@@ -285,14 +285,14 @@ __global__ __launch_bounds__(256) void denoiseFilterViewsPixelKernel(const sgi_b
 }
 
 // pass 1: resA -> resB, pass 2: resB -> resA, pass 3: resA -> reservoirOut; region blocks in view order
-template <int PASS>
+template <int PASS, int R>
 __global__ __launch_bounds__(256) void denoiseFilterViewsKernel(const sgi_batch::ViewDesc* __restrict__ views,
                                                                 int numViews) {
     const int b = (int)xcdSwizzle(blockIdx.x, gridDim.x);
     const sgi_batch::ViewDesc& d = views[sgi_batch::findView<sgi_batch::kFilterBlocks>(views, numViews, b)];
     const float4* in = PASS == 2 ? d.resB : d.resA;
     float4* out = PASS == 1 ? d.resB : (PASS == 2 ? d.resA : (float4*)d.reservoirOut);
-    filterRegion<1 << PASS>(d.g, in, d.normals, out, b - d.dfilterStart);
+    filterRegion<1 << PASS, R>(d.g, in, d.normals, out, b - d.dfilterStart);
 }
 
 // The final pass's temporal blend and combine (vpl_pbr_gi_denoise.fs:336-434) on
@@ -491,12 +491,23 @@ hipError_t taa(const float* screen, const float* prev, const float* velocity, in
     return hipGetLastError();
 }
 
-// Whether the a-trous passes run over columns of four pixels, from the number of 64 x 4 pixel blocks: with
-// one wave or less per SIMD a column's four-fold chain decides, with more its fewer loads do.
-// The whole denoiser by pixels / columns: 320x180 18 / 30 us, 560x315 (711 blocks) 33.3 / 35.1, 640x360
-// (900) 40.3 / 37.2, 960x540 68 / 56.
-constexpr int kColumnBlocks = 800;
-static bool usesColumns(int blocks) { return blocks >= kColumnBlocks; }
+// The three a-trous passes with columns of R pixels (sgi_batch::filterRows).
+template <int R>
+static hipError_t filterPasses(const GbufArgs& g, float4* const* in, float4* const* out, const float4* normals,
+                               hipStream_t s) {
+    const dim3 grid(sgi_batch::filterBlocks(g.W, g.H, R)), block(256);
+    hipLaunchKernelGGL((denoiseFilterKernel<2, R>), grid, block, 0, s, g, in[0], normals, out[0]);
+    hipLaunchKernelGGL((denoiseFilterKernel<4, R>), grid, block, 0, s, g, in[1], normals, out[1]);
+    hipLaunchKernelGGL((denoiseFilterKernel<8, R>), grid, block, 0, s, g, in[2], normals, out[2]);
+    return hipGetLastError();
+}
+template <int R>
+static hipError_t filterPassesViews(const sgi_batch::ViewDesc* views, int numViews, int blocks, hipStream_t s) {
+    hipLaunchKernelGGL((denoiseFilterViewsKernel<1, R>), dim3(blocks), dim3(256), 0, s, views, numViews);
+    hipLaunchKernelGGL((denoiseFilterViewsKernel<2, R>), dim3(blocks), dim3(256), 0, s, views, numViews);
+    hipLaunchKernelGGL((denoiseFilterViewsKernel<3, R>), dim3(blocks), dim3(256), 0, s, views, numViews);
+    return hipGetLastError();
+}
 
 hipError_t denoiseSpatial(const GbufArgs& cur, const FrameArgs& fr, const int32_t* visible, const float* reservoir,
                           float* reservoirOut, const DenoiseBuffers& ws, const int32_t* tiles, bool mergeOnly,
@@ -520,19 +531,15 @@ hipError_t denoiseSpatial(const GbufArgs& cur, const FrameArgs& fr, const int32_
         }
         return e;
     }
-    if (!usesColumns((int)grid.x)) {
-        for (int pass = 0; pass < 3 && e == hipSuccess; ++pass) {
-            hipLaunchKernelGGL(denoiseFilterPixelKernel, grid, block, 0, s, cur, 2 << pass, in[pass], ws.normals,
-                               out[pass]);
-            e = hipGetLastError();
-        }
-        return e;
+    switch (sgi_batch::filterRows((int)grid.x)) {
+        case 1:
+            for (int pass = 0; pass < 3; ++pass)
+                hipLaunchKernelGGL(denoiseFilterPixelKernel, grid, block, 0, s, cur, 2 << pass, in[pass], ws.normals,
+                                   out[pass]);
+            return hipGetLastError();
+        case 2: return filterPasses<2>(cur, in, out, ws.normals, s);
+        default: return filterPasses<4>(cur, in, out, ws.normals, s);
     }
-    const dim3 fgrid(sgi_batch::filterBlocks(cur.W, cur.H));
-    hipLaunchKernelGGL(denoiseFilterKernel<2>, fgrid, block, 0, s, cur, in[0], ws.normals, out[0]);
-    hipLaunchKernelGGL(denoiseFilterKernel<4>, fgrid, block, 0, s, cur, in[1], ws.normals, out[1]);
-    hipLaunchKernelGGL(denoiseFilterKernel<8>, fgrid, block, 0, s, cur, in[2], ws.normals, out[2]);
-    return hipGetLastError();
 }
 
 hipError_t denoiseTemporal(const GbufArgs& cur, const GbufArgs& prev, const FrameArgs& fr, const float* screen,
@@ -569,16 +576,16 @@ hipError_t denoiseViews(const sgi_batch::ViewDesc* views, int numViews, int tota
     hipLaunchKernelGGL(denoiseMergeViewsKernel, dim3(totalBlocks), dim3(256), 0, s, views, numViews, totalBlocks);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    if (usesColumns(totalBlocks)) {
-        hipLaunchKernelGGL(denoiseFilterViewsKernel<1>, dim3(totalFilter), dim3(256), 0, s, views, numViews);
-        hipLaunchKernelGGL(denoiseFilterViewsKernel<2>, dim3(totalFilter), dim3(256), 0, s, views, numViews);
-        hipLaunchKernelGGL(denoiseFilterViewsKernel<3>, dim3(totalFilter), dim3(256), 0, s, views, numViews);
-    } else {
-        for (int pass = 1; pass <= 3; ++pass)
-            hipLaunchKernelGGL(denoiseFilterViewsPixelKernel, dim3(totalBlocks), dim3(256), 0, s, views, numViews,
-                               totalBlocks, pass);
+    switch (sgi_batch::filterRows(totalBlocks)) {
+        case 1:
+            for (int pass = 1; pass <= 3; ++pass)
+                hipLaunchKernelGGL(denoiseFilterViewsPixelKernel, dim3(totalBlocks), dim3(256), 0, s, views, numViews,
+                                   totalBlocks, pass);
+            e = hipGetLastError();
+            break;
+        case 2: e = filterPassesViews<2>(views, numViews, totalFilter, s); break;
+        default: e = filterPassesViews<4>(views, numViews, totalFilter, s); break;
     }
-    e = hipGetLastError();
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(denoiseTemporalViewsKernel, dim3(totalBlocks), dim3(256), 0, s, views, numViews, totalBlocks);
     return hipGetLastError();

@@ -41,8 +41,17 @@ struct ViewDesc {
 
 enum Offset { kTiles = 0, kDirectTiles = 1, kDenoiseBlocks = 2, kFilterBlocks = 3 };
 
-// Blocks of one a-trous filter launch over a W x H view: two for each region of 64 x 32 pixels.
-__host__ __device__ __forceinline__ int filterBlocks(int W, int H) { return ((W + 63) / 64) * ((H + 31) / 32) * 2; }
+// Pixels of a column that a thread of the a-trous filter takes, from the number of 64 x 4 pixel blocks of
+// the launch (a batch: of all views).
+// With few waves a thread's chain decides, with more its loads: the whole denoiser with 1 / 2 / 4 pixels
+// takes 18 / 25 / 30 us at 320x180 (225 blocks), 33.3 / 33.5 / 35.9 at 560x315 (711), 40.2 / 35.2 / 37.2 at
+// 640x360 (900), 54 / 47 / 52 at 800x450 (1469), 69 / 58 / 56 at 960x540 (2025).
+constexpr int kRows2 = 750, kRows4 = 1800;
+inline int filterRows(int blocks) { return blocks < kRows2 ? 1 : (blocks < kRows4 ? 2 : 4); }
+// Blocks of its launch over a W x H view: two for each region of 64 x 8 rows pixels.
+__host__ __device__ __forceinline__ int filterBlocks(int W, int H, int rows) {
+    return ((W + 63) / 64) * ((H + 8 * rows - 1) / (8 * rows)) * 2;
+}
 
 // The view whose work items contain batch item `item` (views are in item order).
 template <int OFF>

@@ -243,7 +243,7 @@ int sgi_views_set(sgi_views* v, int32_t numViews, const sgi_view_io* io, const s
 
     const int ts = v->cfg.tile_size, cap = SGI_MAX_TOTAL_VPLS_PER_FRAME;
     int64_t pix = 0;
-    int tiles = 0, tiles16 = 0, blocks = 0, filter = 0;
+    int tiles = 0, tiles16 = 0, blocks = 0;
     for (int i = 0; i < numViews; ++i) {
         const sgi_view_io& x = io[i];
         const sgi_gbuffer& g = x.gbuffer;
@@ -274,11 +274,9 @@ int sgi_views_set(sgi_views* v, int32_t numViews, const sgi_view_io* io, const s
         d.tileStart = tiles;
         d.dtileStart = tiles16;
         d.dblockStart = blocks;
-        d.dfilterStart = filter;
         tiles += d.tilesX * d.tilesY;
         tiles16 += ((g.width + 15) / 16) * ((g.height + 15) / 16);
         blocks += ((g.width + 63) / 64) * ((g.height + 3) / 4);
-        filter += sgi_batch::filterBlocks(g.width, g.height);
         d.vplUpdated = v->vplUpdated + (size_t)i * cap;
         d.visible = v->visible + (size_t)i * (1 + cap);
         d.entries = v->entries + (size_t)i * cap;
@@ -298,6 +296,12 @@ int sgi_views_set(sgi_views* v, int32_t numViews, const sgi_view_io* io, const s
         d.normals = v->planes + 2 * v->cfg.max_pixels + pix;
         pix += (int64_t)g.width * g.height;
         if (pix > v->cfg.max_pixels) return fail(SGI_E_INVALID, "sgi_views_set: the views exceed max_pixels");
+    }
+    int filter = 0;  // the filter's blocks depend on the whole batch's size
+    for (int i = 0; i < numViews; ++i) {
+        sgi_batch::ViewDesc& d = v->hostDescs[i];
+        d.dfilterStart = filter;
+        filter += sgi_batch::filterBlocks(d.g.W, d.g.H, sgi_batch::filterRows(blocks));
     }
     hipError_t e = hipMemcpyAsync(v->descs, v->hostDescs, (size_t)numViews * sizeof(sgi_batch::ViewDesc),
                                   hipMemcpyHostToDevice, (hipStream_t)stream);

@@ -1,7 +1,7 @@
-"""The a-trous filter at the edges of its regions, in both forms: one pixel per thread below 800 blocks of
-64 x 4 pixels, and from there on (517 x 375 here) a thread filters four pixels of a column that lie a
-lattice step (2, 4, 8) apart, regions are 64 x 32 pixels, and pixels past the frame's last row or column
-have to stay unwritten."""
+"""The a-trous filter at the edges of its regions, in its three forms: one pixel per thread below 750 blocks
+of 64 x 4 pixels, a column of two below 1800 and of four from there on, whose pixels lie a lattice step
+(2, 4, 8) apart in regions of 64 x 16 and 64 x 32.  Pixels past the frame's last row or column have to
+stay unwritten."""
 import numpy as np
 import pytest
 
@@ -15,7 +15,8 @@ pytestmark = pytest.mark.gpu
 REL_L2 = 1e-4  # FP32 images, the bound of every parity test
 
 
-@pytest.mark.parametrize("W,H", [(1, 1), (3, 33), (64, 32), (65, 31), (63, 40), (130, 70), (517, 375), (64, 3203), (2049, 97)])
+@pytest.mark.parametrize("W,H", [(1, 1), (3, 33), (64, 32), (65, 31), (63, 40), (130, 70), (517, 375), (64, 3203), (2049, 97),
+                                 (517, 803), (64, 7201), (2049, 221)])
 def test_denoise_matches_oracle(W, H):
     torch = require_gpu()
     case = Case(small(sc.CORNELL_640x360, name=f"cornell-{W}x{H}-12vpl", width=W, height=H, num_vpls=12,
