@@ -528,6 +528,9 @@ __device__ __forceinline__ void cubeTile(const CubeJob& job, int res, int u, int
             if (first > last || first == kFLOAT_MAX) break;
             const bool now = nearest <= fmaxf(4.0f * first, 4.0f * job.nearPlane) && !(nearest > last);
             uint64_t todo = __ballot(now);
+            // No lane may be taken only where every one compares false: a NaN far plane, nearer than which
+            // nothing is.  Without this the pass would repeat for ever.
+            if (todo == 0) break;
             nearest = now ? kFLOAT_MAX : nearest;
             StagedTri next = lds.stage[__builtin_ctzll(todo)];
             while (todo) {

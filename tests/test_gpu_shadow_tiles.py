@@ -1,7 +1,8 @@
 """The shadow passes' tile drawing at its edges, bit for bit the oracle's brute-force restatement:
 resolutions that end within a region, a tile and a lane's 2x2 texels, one wave per tile and four
 (the calls with many tiles and with few), triangle lists shorter and longer than a wave's scan,
-double-sided meshes (view depths of both signs) and an empty list."""
+double-sided meshes (view depths of both signs), an empty list, and far planes and vertices that are not
+finite."""
 import dataclasses
 
 import numpy as np
@@ -81,3 +82,49 @@ def test_cascades(res, boxes, cull):
     torch.cuda.synchronize()
     want = orc.render_csm(pos, csm, slope=_abi.REFERENCE_CSM_SLOPE_FACTOR, cull=cull)
     assert np.array_equal(depth.cpu().numpy().view(np.uint32), want.view(np.uint32))
+
+
+def _layers(n):
+    """n large triangles one behind the other over +z and -x of the origin, wide in every tile of those faces."""
+    pos = np.zeros((n, 3, 3), np.float32)
+    for k in range(n):
+        z = 2.0 + 0.5 * k
+        pos[k] = [[-3 * z, -2 * z, z], [3 * z, -2 * z, z], [0.1 * k, 4 * z, z]]
+        if k % 4 == 3:
+            pos[k] = pos[k][:, [2, 1, 0]] * np.float32([-1, 1, 1])
+    return pos, (np.arange(n, dtype=np.uint32) * 0x01030507 + 11)
+
+
+# far: every triangle of a wave compares false with a NaN, which nothing is nearer than
+@pytest.mark.parametrize("fmt", [_abi.TEXEL_UNORM16, _abi.TEXEL_F32])
+@pytest.mark.parametrize("far,vertex", [(float("nan"), None), (float("inf"), None), (0.0, None), (-30.0, None),
+                                        (120.0, float("nan")), (120.0, float("inf")), (120.0, -float("inf"))])
+def test_cubes_not_finite(far, vertex, fmt):
+    """Far planes that bound nothing and vertices that are nowhere, with 256 wide triangles in a tile."""
+    torch = require_gpu()
+    pos, col = _layers(256)
+    if vertex is not None:
+        pos[5, 1, 0] = pos[70, 2] = pos[200, 0, 2] = vertex
+    vpls = np.zeros((3, _abi.VPL_FLOATS), np.float32)
+    s, _, _ = _city(1, 3)
+    vpls[:] = s.vpls()[0][:3]
+    vpls[:, 0:3] = [[0, 0, 0], [0.3, -0.2, 0.1], [0, 0, 0]]
+    vpls[:2, 13] = far
+    vpls[2, 13] = 200.0  # a light beside them stays as it is
+    ent = np.stack([np.zeros(3, np.int32), np.arange(3, dtype=np.int32)], 1)
+    res, up = 32, np.arange(3, dtype=np.int32)
+    kinds = {_abi.TEXEL_F32: torch.float32, _abi.TEXEL_UNORM16: torch.int16, None: torch.int32}
+    z, c, cz, cc = _atlases(3, res, fmt, lambda sh, f: torch.full(sh, 3, dtype=kinds[f], device="cuda"))
+    d = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()  # noqa: E731
+    print(f"[tiles] cubes far {far} vertex {vertex} fmt {fmt}", flush=True)
+    GiPass(64, 64).render_vpl_cubes(d(pos), d(col.view(np.int32)), d(vpls), d(up), d(ent), cz, cc,
+                                    cull=_abi.CULLING_NONE)
+    torch.cuda.synchronize()
+    hk = {_abi.TEXEL_F32: np.float32, _abi.TEXEL_UNORM16: np.uint16, None: np.uint32}
+    hz, hc, hcz, hcc = _atlases(3, res, fmt, lambda sh, f: np.zeros(sh, hk[f]))
+    orc.render_vpl_cubes(pos, col, vpls, up, ent, _abi.REFERENCE_VPL_NEAR_PLANE, hcz, hcc, cull=_abi.CULLING_NONE)
+    assert z.cpu().numpy().tobytes() == hz.tobytes()
+    assert np.array_equal(c.cpu().numpy().view(np.uint32), hc)
+    if not far > 0.0:  # the clears
+        assert (hc[:2] == 0xFF000000).all()
+    assert (hc[2] != 0xFF000000).any()
