@@ -238,7 +238,8 @@ int sgi_gbuffer_pack(sgi_ctx* ctx, const sgi_gbuffer* planes, const sgi_gbuffer_
  * atomics, so its order is nondeterministic; ascending order is one of the
  * orders it can produce.)  Needs sgi_set_frame and sgi_set_csm.
  * vplData: device [n]; vplUpdatedData: device [min(n, 4480)] (both 16-byte
- * aligned); visibleIndices: device [1 + min(n, 4480)].  0 <= n <= 10000. */
+ * aligned); visibleIndices: device [1 + min(n, 4480)].  0 <= n <= 10000.
+ * vplUpdatedData may lie over vplData (culling in place, or at any offset). */
 int sgi_cull_global(sgi_ctx* ctx, const sgi_vpl* vplData, int32_t n,
                     sgi_vpl* vplUpdatedData, int32_t* visibleIndices, void* stream);
 
@@ -246,7 +247,7 @@ int sgi_cull_global(sgi_ctx* ctx, const sgi_vpl* vplData, int32_t n,
  * 1675-1701), which reads the visible list back and uploads one atlas entry per
  * visible slot, done on the device: out[s] = shadowIndices[visibleIndices[1 + s]]
  * for s < min(visibleIndices[0], maxCount).  shadowIndices: device [n] by input
- * index; out: device [maxCount]. */
+ * index; out: device [maxCount], which may lie over shadowIndices. */
 int sgi_visible_atlas_entries(sgi_ctx* ctx, const sgi_atlas_entry* shadowIndices,
                               const int32_t* visibleIndices, int32_t maxCount,
                               sgi_atlas_entry* out, void* stream);

@@ -466,17 +466,11 @@ int sgi_render_frame(sgi_ctx* ctx, const sgi_frame_io* io, void* stream) {
         return fail(SGI_E_INVALID, "sgi_render_frame: NULL atlas entry buffer");
     if (io->useTiles && !io->tiles) return fail(SGI_E_INVALID, "sgi_render_frame: tile lists requested, tiles NULL");
     // UpdatePointLights_ -> PerformVirtualPointLightCullingStage1_
-    // with PerformVirtualPointLightCullingStage2_'s atlas entries of the visible slots, unless they
-    // replace the entries they are taken from
+    // with PerformVirtualPointLightCullingStage2_'s atlas entries of the visible slots
     const int maxCount = io->numVpls < SGI_MAX_TOTAL_VPLS_PER_FRAME ? io->numVpls : SGI_MAX_TOTAL_VPLS_PER_FRAME;
-    const bool apart = io->visibleShadowIndices + maxCount <= io->shadowIndices ||
-                       io->shadowIndices + io->numVpls <= io->visibleShadowIndices;
-    int r = cullGlobal(ctx, io->vplData, io->numVpls, io->vplUpdatedData, io->visibleIndices,
-                       apart ? io->shadowIndices : nullptr, io->visibleShadowIndices, stream);
+    int r = cullGlobal(ctx, io->vplData, io->numVpls, io->vplUpdatedData, io->visibleIndices, io->shadowIndices,
+                       io->visibleShadowIndices, stream);
     if (r != SGI_OK) return r;
-    if (!apart && (r = sgi_visible_atlas_entries(ctx, io->shadowIndices, io->visibleIndices, maxCount,
-                                                 io->visibleShadowIndices, stream)) != SGI_OK)
-        return r;
     // PerformVirtualPointLightCullingStage2_: the vplColoring dispatch (vpl_light_color.cs)
     if (io->diffuseCubes &&
         (r = sgi_color_vpls(ctx, io->visibleIndices, io->visibleShadowIndices, io->diffuseCubes, io->cubes,

@@ -54,7 +54,8 @@ __global__ __launch_bounds__(64) void cullVisibilityViewsKernel(const sgi_batch:
 }
 
 // With `all` given, the visible VPLs' atlas entries are written with their records (a frame's and a
-// batch's next launch was that copy: 2 us of a 640x360 frame).
+// batch's next launch was that copy: 2 us of a 640x360 frame).  out NULL: the indices alone.  A wave may
+// write before another has read, so no output may lie over an input (moveVisibleKernel is for those).
 // Stable compaction of the flags: wave ballots and a block prefix, in input
 // order. The block takes kCompactRounds chunks of kCullThreads items at a
 // time: the chunks' flags are loaded together before the one barrier, then
@@ -96,7 +97,7 @@ __device__ __forceinline__ void cullCompactBody(const sgi_vpl* __restrict__ in, 
             const int pos = running + wavePrefix + lanePrefix[k];
             if (f[k] != 0 && pos < SGI_MAX_TOTAL_VPLS_PER_FRAME) {
                 const int i = c0 + k * kCullThreads + (int)threadIdx.x;
-                out[pos] = in[i];
+                if (out) out[pos] = in[i];
                 visible[1 + pos] = i;
                 if (all) entries[pos] = all[i];
             }
@@ -149,7 +150,7 @@ __global__ __launch_bounds__(kSplitThreads) void cullCompactSplitKernel(const sg
         total += before[w] + within[w];
     }
     if (f && pos < SGI_MAX_TOTAL_VPLS_PER_FRAME) {
-        out[pos] = in[i];
+        if (out) out[pos] = in[i];
         visible[1 + pos] = i;
         if (all) entries[pos] = all[i];
     }
@@ -163,6 +164,39 @@ __global__ __launch_bounds__(kCullThreads) void cullCompactViewsKernel(const sgi
     __shared__ int waveCount[kCompactRounds][kCullThreads / 64];
     const sgi_batch::ViewDesc& d = views[blockIdx.x];
     cullCompactBody(in, n, d.visFlags, d.vplUpdated, d.visible, all, d.entries, waveCount);
+}
+
+// The visible slots' records (in -> out, unless in is NULL) and atlas entries (all -> entries, likewise)
+// where an output lies over an input.  One block holds every slot in registers before it writes the first:
+// at most 4480, five a thread, 322 KB of the CU's 512 KB, so any overlap gives what apart buffers do.
+constexpr int kMoveSlots = (SGI_MAX_TOTAL_VPLS_PER_FRAME + kCullThreads - 1) / kCullThreads;
+__global__ __launch_bounds__(kCullThreads) void moveVisibleKernel(const int32_t* __restrict__ visible, int maxCount,
+                                                                  const sgi_vpl* in, sgi_vpl* out,
+                                                                  const sgi_atlas_entry* all,
+                                                                  sgi_atlas_entry* entries) {
+    typedef float Part __attribute__((ext_vector_type(4)));
+    typedef int Entry __attribute__((ext_vector_type(2), aligned(4)));
+    const int count = min(visible[0], maxCount);
+    Part rec[kMoveSlots][4];
+    Entry ent[kMoveSlots];
+#pragma unroll
+    for (int k = 0; k < kMoveSlots; ++k) {
+        const int slot = k * kCullThreads + (int)threadIdx.x;
+        const int i = slot < count ? visible[1 + slot] : 0;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) rec[k][q] = in && slot < count ? reinterpret_cast<const Part*>(in + i)[q] : Part{};
+        ent[k] = all && slot < count ? *reinterpret_cast<const Entry*>(all + i) : Entry{};
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kMoveSlots; ++k) {
+        const int slot = k * kCullThreads + (int)threadIdx.x;
+        if (in && slot < count) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) reinterpret_cast<Part*>(out + slot)[q] = rec[k][q];
+        }
+        if (all && slot < count) *reinterpret_cast<Entry*>(entries + slot) = ent[k];
+    }
 }
 
 __global__ void gatherEntriesKernel(const sgi_atlas_entry* __restrict__ all, const int32_t* __restrict__ visible,
@@ -506,6 +540,12 @@ __global__ __launch_bounds__(64) void cullTilesViewsKernel(const sgi_batch::View
 
 namespace sgi_launch {
 
+// Whether na elements at a and nb at b share memory.
+template <class A, class B>
+static bool overlap(const A* a, int na, const B* b, int nb) {
+    return (uintptr_t)a < (uintptr_t)(b + nb) && (uintptr_t)b < (uintptr_t)(a + na);
+}
+
 hipError_t cullGlobal(const CsmArgs& csm, const FrameArgs& fr, const sgi_vpl* in, int n, sgi_vpl* out,
                       int32_t* visible, uint8_t* flags, const sgi_atlas_entry* all, sgi_atlas_entry* entries,
                       hipStream_t s) {
@@ -514,22 +554,37 @@ hipError_t cullGlobal(const CsmArgs& csm, const FrameArgs& fr, const sgi_vpl* in
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
     }
-    // one block where it takes its items in one round, where out lies over in (it reads before it writes) or
-    // the flags cannot be read by words: 1024 VPLs 5.5 us in one block, 4.7 split
-    const bool apart = out + n <= in || in + n <= out;
-    if (n > kSplitMin && apart && (uintptr_t)flags % 4 == 0)
+    // an output over an input waits for the indices: it is written by moveVisibleKernel, not as the
+    // compaction goes (entries may also take the place of the input records, which are done with by then)
+    const int cap = min(n, SGI_MAX_TOTAL_VPLS_PER_FRAME);
+    const bool moveRecords = overlap(out, cap, in, n);
+    const bool moveEntries = all && (overlap(entries, cap, all, n) || overlap(entries, cap, in, n));
+    sgi_vpl* const out0 = moveRecords ? nullptr : out;
+    const sgi_atlas_entry* const all0 = moveEntries ? nullptr : all;
+    // one block of 1024 threads for a few: 1024 VPLs 5.5 us in one block, 4.7 split
+    if (n > kSplitMin)
         hipLaunchKernelGGL(cullCompactSplitKernel, dim3((n + kSplitThreads - 1) / kSplitThreads), dim3(kSplitThreads),
-                           0, s, in, n, flags, out, visible, all, entries);
+                           0, s, in, n, flags, out0, visible, all0, entries);
     else
-        hipLaunchKernelGGL(cullCompactKernel, dim3(1), dim3(kCullThreads), 0, s, in, n, flags, out, visible, all,
+        hipLaunchKernelGGL(cullCompactKernel, dim3(1), dim3(kCullThreads), 0, s, in, n, flags, out0, visible, all0,
                            entries);
+    if (moveRecords || moveEntries)
+        hipLaunchKernelGGL(moveVisibleKernel, dim3(1), dim3(kCullThreads), 0, s, visible, cap,
+                           moveRecords ? in : nullptr, out, moveEntries ? all : nullptr, entries);
     return hipGetLastError();
 }
 
 hipError_t gatherVisibleEntries(const sgi_atlas_entry* all, const int32_t* visible, int maxCount, sgi_atlas_entry* out,
                                 hipStream_t s) {
     if (maxCount <= 0) return hipSuccess;
-    hipLaunchKernelGGL(gatherEntriesKernel, dim3((maxCount + 255) / 256), dim3(256), 0, s, all, visible, maxCount, out);
+    // how many entries `all` holds is not given: as many as there may be VPLs, so an output close behind goes
+    // the safe way too (64 slots 1.7 -> 2.2 us, 4096 1.7 -> 3.3)
+    if (overlap(out, maxCount, all, SGI_MAX_TOTAL_VPLS_BEFORE_CULLING))
+        hipLaunchKernelGGL(moveVisibleKernel, dim3(1), dim3(kCullThreads), 0, s, visible, maxCount, nullptr, nullptr,
+                           all, out);
+    else
+        hipLaunchKernelGGL(gatherEntriesKernel, dim3((maxCount + 255) / 256), dim3(256), 0, s, all, visible, maxCount,
+                           out);
     return hipGetLastError();
 }
 
