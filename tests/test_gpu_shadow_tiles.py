@@ -128,3 +128,45 @@ def test_cubes_not_finite(far, vertex, fmt):
     if not far > 0.0:  # the clears
         assert (hc[:2] == 0xFF000000).all()
     assert (hc[2] != 0xFF000000).any()
+
+
+def test_every_light_of_a_call_in_batches():
+    """24012 triangles: a call of 500 lights runs in several batches (48 B a triangle and light within 256 MB:
+    232 lights).  Every light's cube is the one that a call of 50 lights, a single batch, gives it; those next
+    to the boundaries are the oracle's."""
+    torch = require_gpu()
+    s = sc.Scene(dataclasses.replace(sc.CITY_1080P, num_vpls=500))
+    pos, col = s.triangles()
+    batch = (64 << 20) // (12 * ((pos.shape[0] + 3) // 4 * 4) + 6)
+    assert pos.shape[0] == 24012 and batch == 232
+    vpls, _ = s.vpls()
+    ent = np.stack([np.arange(500) // 250, np.arange(500) % 250], 1).astype(np.int32)
+    d = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()  # noqa: E731
+
+    def atlases(alloc):  # 250 cubes in each of two
+        z, c, cz, cc = _atlases(250, 16, _abi.TEXEL_UNORM16, lambda sh, f: alloc((2,) + sh, f))
+        for a in (cz, cc):
+            a.num_atlases = 2
+            t = z if a is cz else c
+            a.atlas[1] = t[1].ctypes.data if isinstance(t, np.ndarray) else t[1].data_ptr()
+        return z, c, cz, cc
+
+    dp, dc, dv, de, gi = d(pos), d(col.view(np.int32)), d(vpls), d(ent), GiPass(64, 64)
+    got = []
+    for step in (500, 50):
+        z, c, cz, cc = atlases(lambda sh, f: torch.full(sh, 3, dtype=torch.int32 if f is None else torch.int16,
+                                                        device="cuda"))
+        print(f"[tiles] 500 lights, {step} a call", flush=True)
+        for first in range(0, 500, step):
+            gi.render_vpl_cubes(dp, dc, dv, d(np.arange(first, first + step, dtype=np.int32)), de, cz, cc)
+        torch.cuda.synchronize()
+        got.append([t.view(500, 6, 16, 16).cpu().numpy() for t in (z, c)])
+    for one, few in zip(*got):
+        assert np.array_equal(one, few), np.nonzero((one != few).any(axis=(1, 2, 3)))[0]
+    hz, hc, hcz, hcc = atlases(lambda sh, f: np.zeros(sh, np.uint32 if f is None else np.uint16))
+    pick = np.array([batch - 1, batch, 2 * batch - 1, 2 * batch, 499], np.int32)
+    orc.render_vpl_cubes(pos, col, vpls, pick, ent, _abi.REFERENCE_VPL_NEAR_PLANE, hcz, hcc)
+    z, c = got[0]
+    for u in pick:
+        assert z[u].tobytes() == hz.reshape(500, 6, 16, 16)[u].tobytes(), f"distance of light {u}"
+        assert np.array_equal(c.view(np.uint32)[u], hc.reshape(500, 6, 16, 16)[u]), f"colour of light {u}"
