@@ -64,3 +64,41 @@ def test_tonemap_cornell_frame():
     _check(fb.combined.cpu().numpy(), out.cpu().numpy().view(np.uint32), 2.2)
     with pytest.raises(_abi.SgiError):
         gi.tonemap(fb.combined, out, gamma=0.0)
+
+
+def _near_ties(gamma, steps):
+    """Lit values whose stored value lies at k + 1/2 codes, and up to `steps` ulp beside them."""
+    v = (np.arange(255) + 0.5) / 255.0
+    film = v ** gamma
+    # (2.51 x^2 + 0.03 x) / (2.43 x^2 + 0.59 x + 0.14) = film
+    a, b, c = 2.51 - 2.43 * film, 0.03 - 0.59 * film, -0.14 * film
+    x = (-2.0 * c / (b + np.sqrt(b * b - 4.0 * a * c))).astype(np.float32)
+    return (x.view(np.int32)[:, None] + np.arange(-steps, steps + 1)).astype(np.int32).view(np.float32)
+
+
+# 1 / gamma: below 1, 1 (the estimate's least margin), up to 16 (its margin grows with it), and above (exact form)
+@pytest.mark.parametrize("gamma", [1.0, 2.2, 0.45, 0.07, 0.0625, 0.05, 8.0])
+def test_tonemap_margins(gamma):
+    """Every power the estimate serves, and those it leaves to the exact form: over random values, and beside
+    every code's tie, where the estimate may not decide."""
+    torch = require_gpu()
+    rng = np.random.default_rng(7)
+    ties = _near_ties(gamma, 400)
+    rows = -(-ties.size // (3 * 317)) + 60
+    lit = np.exp(rng.uniform(np.log(1e-4), np.log(100.0), (rows, 317, 3))).astype(np.float32)
+    lit.reshape(-1)[:ties.size] = ties.reshape(-1)
+    lit[-1, :9, 0] = [0.0, -0.0, -1e-3, -5.0, 1e9, 2e9, 1e20, np.inf, np.nan]
+    gi = GiPass(317, rows, 16, 12)
+    out = torch.zeros((rows, 317), dtype=torch.int32, device="cuda")
+    gi.tonemap(torch.from_numpy(lit).cuda(), out, gamma=gamma)
+    torch.cuda.synchronize()
+    got = out.cpu().numpy().view(np.uint32)
+    want, film = orc.tonemap(lit, gamma)
+    gc, wc = (np.stack([(t >> (8 * k)) & 0xFF for k in range(3)], -1).astype(np.int64) for t in (got, want))
+    diff = gc != wc
+    v = film.astype(np.float64) * 255.0
+    tie = np.abs(v - (np.floor(v) + 0.5))
+    near = tie <= 8 * 255.0 * np.spacing(np.maximum(film, 1e-30))  # the two pows' distance, as above
+    print(f"[tonemap] gamma {gamma}: {int(diff.sum())} of {diff.size} codes differ, {int(near.sum())} near a tie",
+          flush=True)
+    assert near.sum() > 255 and np.all(near[diff]) and np.all(np.abs(gc - wc)[diff] == 1)
