@@ -180,3 +180,62 @@ def test_fp8_quality_on_city(lib):
         rel[name] = float(((x - target) ** 2 / (target * target + 1e-2)).mean())
     print(f"[fp8 quality] relMSE bf16 {rel['bf16']:.6f} fp8 {rel['fp8']:.6f}", flush=True)
     assert rel["fp8"] <= 1.05 * rel["bf16"]
+
+
+def _exact_params(rng):
+    """A network whose sums FP32 holds exactly, so that no E4M3 rounding can fall to the other side: three
+    weights of 1/2 (one of 1 over the BF16 features) and a bias a channel, of either sign, at any tap."""
+    p = np.zeros(kpcn.PARAMS, np.float32)
+    for l in range(kpcn.LAYERS):
+        w = np.zeros((9, kpcn.C, kpcn.C), np.float32)
+        for o in range(kpcn.C):
+            if l == 0:
+                w[rng.integers(0, 9), o, rng.integers(0, 10)] = rng.choice([-1.0, 1.0])
+            else:
+                for _ in range(3):
+                    w[rng.integers(0, 9), o, rng.integers(0, kpcn.C)] = rng.choice([-0.5, 0.5, 0.5])
+        b = rng.integers(-4, 9, kpcn.C).astype(np.float32) / 8.0
+        p[l * kpcn.LAYER_PARAMS:(l + 1) * kpcn.LAYER_PARAMS] = np.concatenate([w.reshape(-1), b])
+    return p
+
+
+# sides that cut a tile, with odd levels below (the pooling's last row and column, the upsampling's clamp)
+@pytest.mark.parametrize("H,W", [(33, 31), (50, 67), (48, 64), (1, 70), (17, 15)])
+def test_fp8_network_edges(lib, H, W):
+    """The FP8 network where tiles are cut, against the oracle: with the shipped weights a sum may fall to
+    either side of a rounding tie and the layers after it carry that on over the whole image, so a wrong
+    column could hide; here every stored activation is the oracle's, and the reconstruction, FP32 against
+    64 bits, holds the bound of the FP32 images, inside and in the last columns and rows by themselves."""
+    torch = require_gpu()
+    rng = np.random.default_rng(H * W)
+    case = Case(dataclasses.replace(sc.CORNELL_640x360, name=f"cornell-{W}x{H}-8vpl", width=W, height=H, num_vpls=8,
+                                    cube_res=16, csm_res=64))
+    gi = GiPass(W, H, 16, 12)
+    gi.set_frame(case.dev.frame)
+    gi.set_csm(case.dev.csm_struct())
+    f32 = dict(dtype=torch.float32, device="cuda")
+    lit, col = (torch.from_numpy(rng.uniform(0.1, 2, (H, W, 3)).astype(np.float32)).cuda() for _ in range(2))
+    res = torch.from_numpy(rng.uniform(0.1, 2, (H, W, 4)).astype(np.float32)).cuda()
+    g = case.dev.gbuffer()
+    params = _exact_params(rng)
+    wts = kpcn.Weights(params)
+    S, Cs = np.ones((kpcn.LEVELS - 1, kpcn.C)), np.ones((kpcn.LEVELS, kpcn.C))
+    f8 = kpcn_fp8.Fp8Net(wts, *kpcn_fp8.quantize(params, S, Cs))
+    feat, rad = torch.empty((H, W, 32), dtype=torch.bfloat16, device="cuda"), torch.empty((H, W, 3), **f32)
+    gi.kpcn_features(g, res, feat, rad)
+    outs = [torch.zeros((H, W, c), **f32) for c in (3, 3, 4)] + [torch.zeros((H, W), **f32)]
+    vis = torch.tensor([8], dtype=torch.int32, device="cuda")
+    gi.denoise_learned(g, None, vis, lit, col, res, None, None, f8.net(), float("inf"), gi.kpcn_workspace(), *outs)
+    torch.cuda.synchronize()
+    got = outs[2][..., :3].cpu().numpy().astype(np.float64)
+    featn, radn = feat.float().cpu().numpy().astype(np.float64), rad.cpu().numpy().astype(np.float64)
+    net = ko.NetF8(params, S, Cs)
+    want = ko.reconstruct(net.forward(featn), radn)[0][0]
+    alive = [np.count_nonzero(net.a[k]) / net.a[k].size for k in sorted(net.a)]
+    print(f"[fp8 net] {W}x{H}: {min(alive):.2f} .. {max(alive):.2f} of an activation's values are not zero", flush=True)
+    assert min(alive) > 0.2
+    last = slice(-2, None)
+    for part, at in (("whole", (slice(None), slice(None))), ("columns", (slice(None), last)), ("rows", (last,))):
+        e = np.linalg.norm(got[at] - want[at]) / np.linalg.norm(want[at])
+        print(f"[fp8 net] {W}x{H} {part}: rel-L2 {e:.2e}", flush=True)
+        assert e <= 1e-4, part
