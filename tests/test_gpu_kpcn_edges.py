@@ -91,3 +91,29 @@ def test_fused_network_is_the_training_path(H, W):
     want = kpcn.Trainer(wts, H, W).forward(feat, rad)
     torch.cuda.synchronize()
     assert torch.equal(outs[2][..., :3], want)
+
+
+def test_gradients_of_samples_add():
+    """Two samples without zero_grad between them leave the sum of their gradients: one addition a parameter."""
+    torch = require_gpu()
+    H, W = 40, 56
+    rng = np.random.default_rng(9)
+    tr = kpcn.Trainer(kpcn.Weights(kpcn.init_params(7)), H, W)
+    samples = []
+    for _ in range(2):
+        feat = np.zeros((H, W, 32))
+        feat[..., :10] = rng.normal(0, 1, (H, W, 10))
+        rad, target = (torch.from_numpy(rng.uniform(0.1, 2, (H, W, 3)).astype(np.float32)).cuda() for _ in range(2))
+        samples.append((_bf(torch, feat), rad, target))
+
+    def run(which):
+        tr.zero_grad()
+        for feat, rad, target in which:
+            tr.forward(feat, rad)
+            tr.loss_backward(target, err_weight=0.1)
+        torch.cuda.synchronize()
+        return tr.grad.clone()
+
+    first, second = run(samples[:1]), run(samples[1:])
+    assert not torch.equal(first, second) and bool((first != 0).any()) and bool((second != 0).any())
+    assert torch.equal(run(samples), first + second)
