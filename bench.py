@@ -42,7 +42,8 @@ Inputs are
 generated on the GPU before the timed regions; the denoiser history alternates
 between two buffer sets as the reference swaps its FBOs.
 
-Prints one JSON line.  With the default flags it also times the CPU oracle
+Prints one JSON line, without the points of the sweeps (they are on stderr as they
+are timed; --details FILE holds everything).  With the default flags it also times the CPU oracle
 (16 host threads) on a bounded sample of the a-trous frame at the learned
 operating point's equal-relMSE sample count as the CPU baseline.
 """
@@ -58,6 +59,13 @@ sys.path.insert(0, HERE)
 
 METRIC = "1080p GI frames/s, learned vs à-trous denoise at equal relMSE to converged"
 HBM_PEAK_GBS = 8000.0
+# Kept out of the printed line, which a reader may hold only the last 12 KB of: with them it has 34 KB.
+SWEEPS = ("learned_sweep", "learned_1024_vpls", "learned_1024_sweep", "atrous_1024_sweep", "atrous_sweep")
+
+
+def line_of(result):
+    """The printed JSON line of a whole result."""
+    return json.dumps({k: v for k, v in result.items() if k not in SWEEPS})
 
 
 def parse():
@@ -92,6 +100,7 @@ def parse():
     ap.add_argument("--cpu-rows", type=int, default=120, help="image rows of the CPU baseline sample")
     ap.add_argument("--cpu-threads", type=int, default=min(16, os.cpu_count() or 1),
                     help="host threads of the CPU baseline (the oracle's rows split over them)")
+    ap.add_argument("--details", default=None, metavar="FILE", help="write the whole result, sweeps included, to FILE")
     ap.add_argument("--copy-probe-mb", type=int, default=0,
                     help="instead of the benchmark, run a plain device copy of this many MiB (counter calibration)")
     return ap.parse_args()
@@ -1134,7 +1143,10 @@ def main():
             bl = (learned_res["samples_per_pixel"], (f8net.net() if learned_res["network_precision"] == "fp8"
                                                       else wts.net()), threshold, learned_res["network_precision"])
         result["batched_views"] = batched_views(args, bl)
-    print(json.dumps(result), flush=True)
+    if args.details:
+        with open(args.details, "w") as f:
+            json.dump(result, f, indent=1)
+    print(line_of(result), flush=True)
 
 
 if __name__ == "__main__":
