@@ -25,7 +25,7 @@
 // and appends the triangle to each face it can overlap (one atomic per block
 // and face), with the 32x32-texel regions its projection can touch; (2) each
 // 16x16 tile of a face is drawn by one wave (or by four, each a quarter of the
-// list, where the call's tiles are too few to fill the chip): the wave picks
+// list, where it is long and the tiles are few): the wave picks
 // its triangles from the face list by integer range tests (4 B per triangle),
 // sets up 64 at a time (edge vectors in face axes), draws those of a few
 // texels one texel per lane into LDS, and tests its texels, 2x2 per lane,
@@ -900,11 +900,19 @@ __global__ __launch_bounds__(64 * SLICES, 4) void csmRasterKernel(CsmJob job, in
     }
 }
 
-// Tiles below which each is drawn by a whole block: one wave per tile then leaves most of the chip's
-// 1024 SIMDs waiting for the few tiles that hold many triangles (7680 tiles: 0.215 ms by waves, 0.139
-// by blocks; 16384 cascade tiles: 0.238 and 0.184), and a block per tile repeats the tile's setup
-// (147456 tiles: 0.94 ms by waves, 1.60 by blocks).
-constexpr long kFewTiles = 32768;
+// Whether a tile is drawn by a whole block that shares its list, or by one wave.  A block shortens a long
+// list's chain, which the launch waits for, and repeats the tile's setup; both grow, the first with the
+// triangles and the second with the tiles, and they are equal about where there are 3 triangles to 4 tiles
+// (us by waves / by blocks).  Cubes: 1212 triangles, 7680 tiles 70 / 95; 4812, 1536 91 / 71, 7680 112 / 115,
+// 18432 126 / 177; 12012, 7680 132 / 115, 18432 150 / 186; 24012, 7680 208 / 137, 30720 360 / 337, 49152
+// 373 / 495, 147456 850 / 1343; 96012, 46080 1683 / 1287, 147456 3898 / 3592.  Cascades: 12012, 4096 91 / 57,
+// 16384 105 / 107, 30976 143 / 177; 96012, 33856 992 / 932, 141376 3163 / 3346.  Up to `spare` tiles, one
+// wave each would leave SIMDs idle: cascades of 4096, 516 triangles 32 / 32, 2412 65 / 41 (cubes' lists,
+// of six faces, are shorter: 0).  A list within one scan is the first wave's alone: 516, the cubes of 15
+// lights 83 / 155.  (A launch holds fewer than 2^32 threads.)
+static bool drawnByBlocks(long tiles, int count, long spare) {
+    return count > kScan && tiles < 1L << 23 && (tiles <= spare || tiles * 3 < (long)count * 4);
+}
 
 }  // namespace
 
@@ -935,7 +943,7 @@ hipError_t renderCsm(const float* pos, int count, int keepSign, float slope, int
         hipLaunchKernelGGL(csmListKernel, dim3((unsigned)((count + kListBlock - 1) / kListBlock), SGI_NUM_CASCADES),
                            dim3(kListBlock), 0, s, job, rpe);
     const long tiles = 4L * SGI_NUM_CASCADES * rpe * rpe;
-    if (tiles < kFewTiles)
+    if (drawnByBlocks(tiles, count, 4096))
         hipLaunchKernelGGL(csmRasterKernel<4>, dim3((unsigned)tiles), dim3(256), 0, s, job, rpe, depth);
     else
         hipLaunchKernelGGL(csmRasterKernel<1>, dim3((unsigned)tiles), dim3(64), 0, s, job, rpe, depth);
@@ -967,7 +975,7 @@ hipError_t renderVplCubes(const float* pos, const uint32_t* colors, int count, i
         const int wc = withDiffuse ? 1 : 0;
         const long tiles = 4L * batch * 6 * rpe * rpe;
 #define SGI_CUBE_RASTER(F)                                                                                            \
-    if (tiles < kFewTiles)                                                                                            \
+    if (drawnByBlocks(tiles, count, 0))                                                                               \
         hipLaunchKernelGGL((cubeRasterKernel<F, 4>), dim3((unsigned)tiles), dim3(256), 0, s, job, res, rpe, dist, diffuse, wc); \
     else                                                                                                              \
         hipLaunchKernelGGL((cubeRasterKernel<F, 1>), dim3((unsigned)tiles), dim3(64), 0, s, job, res, rpe, dist, diffuse, wc)

@@ -84,6 +84,12 @@ def test_cascades(res, boxes, cull):
     assert np.array_equal(depth.cpu().numpy().view(np.uint32), want.view(np.uint32))
 
 
+# lists within one scan and just beyond it, and either side of 3 triangles to 4 tiles
+@pytest.mark.parametrize("res,lights,boxes", [(40, 2, 41), (40, 2, 42), (64, 8, 50), (64, 9, 50)])
+def test_cubes_at_the_lines_between_the_forms(res, lights, boxes):
+    test_cubes(res, lights, boxes, _abi.TEXEL_UNORM16, _abi.CULLING_NONE)
+
+
 def _layers(n):
     """n large triangles one behind the other over +z and -x of the origin, wide in every tile of those faces."""
     pos = np.zeros((n, 3, 3), np.float32)
