@@ -34,7 +34,8 @@
 // LESS rule.  Culling is conservative (region margins as the frustum test's
 // 2^-12, edge margins from the rounding bound of the edge functions); the
 // per-texel test alone decides every value, in the restatement's operation
-// order (-ffp-contract=off).
+// order (-ffp-contract=off).  A mesh of a few triangles takes one launch without
+// lists (cubeShortKernel).
 //
 // What bounds it: the latency of a wave's serial triangles, then VALU issue.
 // Towards the horizon a region holds more than a thousand triangles of a few
@@ -335,6 +336,32 @@ __device__ __forceinline__ float4 faceAxes(bool neg, f3 C, float w) {
     else return make_float4(neg ? -C.z : C.z, neg ? -C.x : C.x, -C.y, w);
 }
 
+// Bound on a computed edge function's distance from the exact one: two products per cross component and
+// three per dot product of vertices at most this far away, |ray| < 2.
+__device__ __forceinline__ float edgeError(f3 a, f3 b, f3 c) {
+    return 0x1p-20f * gmax(dot(a, a), gmax(dot(b, b), dot(c, c)));
+}
+
+// A lower bound of the view depth of the triangle's fragments among rays within h of (midS, midT) on each
+// axis, kFLOAT_MAX where it has none.  A fragment needs e0, e1, e2 all of V's sign (or zero): the view depth
+// V / (e0 + e1 + e2) is positive.  So a rectangle over which one edge, after V's sign, stays below -4 err
+// has no fragment, and where there are some their view depth is at least |V| over the largest sum of the
+// edges.
+__device__ __forceinline__ float nearestDepth(const float4* e, float V, float err, float midS, float midT, float h,
+                                              float farP) {
+    const float sg = V < 0.0f ? -1.0f : 1.0f;
+    float most = 0.0f;
+    bool out = false;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        const float top = sg * (e[i].x + midS * e[i].y + midT * e[i].z) + (fabsf(e[i].y) + fabsf(e[i].z)) * h;
+        out = out || top < -4.0f * err;
+        most += top + 4.0f * err;
+    }
+    const float t = fabsf(V) * frcp(most) * (1.0f - 0x1p-12f);
+    return out ? kFLOAT_MAX : (most > 1e-30f && t < farP ? t : (most > 1e-30f ? farP : 0.0f));
+}
+
 struct CubeLds {
     int32_t cand[kCand];
     StagedTri stage[64];
@@ -451,24 +478,9 @@ __device__ __forceinline__ void cubeTile(const CubeJob& job, int res, int u, int
             const float4 e[3] = {faceAxes<AXIS>(neg, C0, V), faceAxes<AXIS>(neg, C1, __int_as_float(k)),
                                  faceAxes<AXIS>(neg, C2, tiny ? 0.0f : V)};
             lds.stage[lane] = StagedTri{e[0], e[1], e[2]};
-            // A fragment needs e0, e1, e2 all of V's sign (or zero): the view depth V / (e0 + e1 + e2)
-            // is positive.  The computed e_k lie within err = 2^-20 max |vertex|^2 of the exact ones
-            // (two products per cross component, three per dot product, |ray| < 2).  So a tile over
-            // which one edge, after V's sign, stays below -4 err has no fragment, and where there are
-            // some their view depth is at least |V| over the largest sum of the edges.
-            const float err = 0x1p-20f * gmax(dot(a, a), gmax(dot(b, b), dot(c, c)));
-            const float sg = V < 0.0f ? -1.0f : 1.0f;
-            float most = 0.0f;
-            bool out = false;
-#pragma unroll
-            for (int i = 0; i < 3; ++i) {
-                const float top = sg * (e[i].x + midS * e[i].y + midT * e[i].z) + (fabsf(e[i].y) + fabsf(e[i].z)) * h;
-                out = out || top < -4.0f * err;
-                most += top + 4.0f * err;
-            }
-            if (!out) {
-                const float t = fabsf(V) * frcp(most) * (1.0f - 0x1p-12f);
-                nearest = most > 1e-30f && t < farP ? t : (most > 1e-30f ? farP : 0.0f);
+            const float err = edgeError(a, b, c);
+            nearest = nearestDepth(e, V, err, midS, midT, h, farP);
+            if (nearest != kFLOAT_MAX) {
                 float m[3], s[3], t3[3];
 #pragma unroll
                 for (int i = 0; i < 3; ++i) {
@@ -621,6 +633,159 @@ __global__ __launch_bounds__(64 * SLICES, 4) void cubeRasterKernel(CubeJob job, 
         case 0: cubeTile<FMT, 0, SLICES>(job, res, u, f, x0, y0, slice, zb, cb, lds[slice], tile); break;
         case 1: cubeTile<FMT, 1, SLICES>(job, res, u, f, x0, y0, slice, zb, cb, lds[slice], tile); break;
         default: cubeTile<FMT, 2, SLICES>(job, res, u, f, x0, y0, slice, zb, cb, lds[slice], tile); break;
+    }
+}
+
+// The whole pass for a mesh of at most kShort triangles: a block per 32x32 region tests them all against the
+// region's sub-frustum, a triangle per thread, stages those that may touch it in their order, and draws them
+// with exact keys at every texel, 2x2 per lane.  More than kDeep are drawn near ones first, until the next
+// one lies behind every texel of the wave.
+// One launch and no lists: over few triangles the lists' latency and each tile's setup are most of the time.
+// GPU us by lists and tiles / this, 84 triangles of a room: 5 lights of 256^2 33 / 19, 64 lights 184 / 106,
+// 300 lights of 64^2 83 / 50; 252 of a city, 96 lights of 256^2 237 / 184.  (256 triangles that all cover
+// one another are the tiles' case, 1616 / 1930, but few meshes of that size are.)
+constexpr int kShort = 256, kDeep = 16;
+struct ShortLds {
+    StagedTri stage[kShort];
+    float nearest[kShort];
+    uint8_t order[kShort];
+    int waveCount[kShort / 64];
+};
+
+template <int FMT, int AXIS>
+__device__ __forceinline__ void cubeRegion(const CubeJob& job, int res, int u, int f, int x0, int y0, void* zb,
+                                           uint32_t* cb, ShortLds& lds) {
+    const sgi_vpl& v = job.vpls[job.updates[job.first + u]];
+    const f3 L{v.position[0], v.position[1], v.position[2]};
+    const float farP = v.farPlane;
+    const bool neg = (f & 1) != 0;
+    const int k = (int)threadIdx.x, lane = k & 63, wave = k >> 6;
+    bool keep = false;
+    float nearest = kFLOAT_MAX;
+    StagedTri tri{};
+    if (k < job.count) {
+        const f3 a = vertexRel(job.pos, k, 0, L), b = vertexRel(job.pos, k, 1, L), c = vertexRel(job.pos, k, 2, L);
+        const f3 C0 = cross3(b, c);
+        const float V = dot(a, C0);
+        if (!culledFromLight(job.cull, V)) {
+            const float4 q[3] = {faceAxes<AXIS>(neg, a, 0.0f), faceAxes<AXIS>(neg, b, 0.0f), faceAxes<AXIS>(neg, c, 0.0f)};
+            const float m[3] = {q[0].x, q[1].x, q[2].x}, s[3] = {q[0].y, q[1].y, q[2].y}, t[3] = {q[0].z, q[1].z, q[2].z};
+            const auto edge = [&](int i) { return 2.0f * (float)i / (float)res - 1.0f; };
+            const float4 e[3] = {faceAxes<AXIS>(neg, C0, V), faceAxes<AXIS>(neg, cross3(c, a), __int_as_float(k)),
+                                 faceAxes<AXIS>(neg, cross3(a, b), 0.0f)};
+            nearest = nearestDepth(e, V, edgeError(a, b, c), edge(x0 + kRegion / 2), edge(y0 + kRegion / 2),
+                                   (float)(kRegion - 1) / (float)res, farP);
+            keep = nearest != kFLOAT_MAX &&
+                   !outsideFrustum(m, s, t, edge(x0), edge(min(x0 + kRegion, res)), edge(y0),
+                                   edge(min(y0 + kRegion, res)), job.nearPlane, farP);
+            tri = StagedTri{e[0], e[1], e[2]};
+        }
+    }
+    const uint64_t bal = __ballot(keep);
+    if (lane == 0) lds.waveCount[wave] = __popcll(bal);
+    __syncthreads();
+    int at = __popcll(bal & ((1ull << lane) - 1ull)), total = 0;
+#pragma unroll
+    for (int w = 0; w < kShort / 64; ++w) {
+        at += w < wave ? lds.waveCount[w] : 0;
+        total += lds.waveCount[w];
+    }
+    if (keep) {
+        lds.stage[at] = tri;
+        lds.nearest[at] = nearest;
+    }
+    __syncthreads();
+    const int i0 = x0 + (k & 15) * 2, j0 = y0 + (k >> 4) * 2;
+    float s[2], t[2], len[4], depth[4];
+    uint32_t best[4];
+    int drawn[4];
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+        s[p] = 2.0f * ((float)(i0 + p) + 0.5f) / (float)res - 1.0f;
+        t[p] = 2.0f * ((float)(j0 + p) + 0.5f) / (float)res - 1.0f;
+    }
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+        len[p] = rayLength<AXIS>(s[p & 1], t[p >> 1]);
+        depth[p] = farP * frcp(len[p]);  // of the clear
+        best[p] = depthKey<FMT>(1.0f);   // the depth clear (:1455-1456)
+        drawn[p] = -1;                   // the colour clear (:1453-1454)
+    }
+    const auto draw = [&](const StagedTri& st) __attribute__((always_inline)) {
+        const float4 a = st.c0, b = st.c1, c = st.c2;
+        const int index = __float_as_int(b.w);
+#pragma unroll
+        for (int p = 0; p < 4; ++p) {
+            const float e0 = edgeAt<AXIS>(a.x, a.y, a.z, s[p & 1], t[p >> 1]);
+            const float e1 = edgeAt<AXIS>(b.x, b.y, b.z, s[p & 1], t[p >> 1]);
+            const float e2 = edgeAt<AXIS>(c.x, c.y, c.z, s[p & 1], t[p >> 1]);
+            // >= 0 where the edges agree in sign; NaN edges give a NaN depth, never drawn
+            const float in = fmaxf(fminf(fminf(e0, e1), e2), -fmaxf(fmaxf(e0, e1), e2));
+            const float den = e0 + e1 + e2;
+            if (in < 0.0f || den == 0.0f) continue;
+            const float tv = a.w / den;
+            if (!(tv >= job.nearPlane && tv <= farP)) continue;  // GL clipping to [near, far]
+            const uint32_t key = depthKey<FMT>((tv * len[p]) / farP);
+            if (key < best[p] || (key == best[p] && index < drawn[p])) {
+                best[p] = key;
+                drawn[p] = index;
+                depth[p] = tv;
+            }
+        }
+    };
+    if (total <= kDeep) {
+        for (int q = 0; q < total; ++q) draw(lds.stage[q]);
+    } else {
+        if (k < total) {  // its place among the depths (their bits: NaN too has one)
+            const uint32_t mine = __float_as_uint(lds.nearest[k]);
+            int place = 0;
+            for (int q = 0; q < total; ++q) {
+                const uint32_t other = __float_as_uint(lds.nearest[q]);
+                place += other < mine || (other == mine && q < k) ? 1 : 0;
+            }
+            lds.order[place] = (uint8_t)k;
+        }
+        __syncthreads();
+        const float invFar = frcp(farP);
+        for (int q = 0; q < total; ++q) {
+            const int n = lds.order[q];
+            const float near = lds.nearest[n];
+            bool behind = true;  // of what every texel holds, by more than a key's step (NaN: it may not be)
+#pragma unroll
+            for (int p = 0; p < 4; ++p)
+                behind = behind &&
+                         near > depth[p] + keyCell<FMT>(depth[p] * len[p] * invFar) * 1.01f * farP * frcp(len[p]);
+            if (!__ballot(!behind)) break;
+            draw(lds.stage[n]);
+        }
+    }
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+        const int i = i0 + (p & 1), j = j0 + (p >> 1);
+        if (i >= res || j >= res) continue;
+        const size_t o = ((size_t)f * res + j) * res + i;
+        if constexpr (FMT == SGI_TEXEL_F32) ((float*)zb)[o] = __uint_as_float(best[p]);
+        else ((uint16_t*)zb)[o] = (uint16_t)best[p];
+        if (cb) cb[o] = (drawn[p] < 0 ? 0u : job.colors[drawn[p]]) | 0xFF000000u;
+    }
+}
+
+template <int FMT>
+__global__ __launch_bounds__(kShort) void cubeShortKernel(CubeJob job, int res, int regionsPerEdge, CubeArgs dist,
+                                                          CubeArgs diffuse, int withColor) {
+    __shared__ ShortLds lds;
+    const int perFace = regionsPerEdge * regionsPerEdge;
+    const int r = blockIdx.x % perFace, f = (blockIdx.x / perFace) % 6, u = blockIdx.x / (perFace * 6);
+    const int x0 = r % regionsPerEdge * kRegion, y0 = r / regionsPerEdge * kRegion;
+    const sgi_atlas_entry e = job.entries[job.updates[job.first + u]];
+    // an entry outside the atlases names no cube: nothing is written for it
+    if (e.index < 0 || e.index >= dist.numAtlases || e.layer < 0 || e.layer >= dist.layers) return;
+    void* zb = const_cast<void*>(cubeLayerBase(dist, e.index, e.layer, texelBytes(FMT)));
+    uint32_t* cb = withColor ? (uint32_t*)const_cast<void*>(cubeLayerBase(diffuse, e.index, e.layer, 4)) : nullptr;
+    switch (f >> 1) {
+        case 0: cubeRegion<FMT, 0>(job, res, u, f, x0, y0, zb, cb, lds); break;
+        case 1: cubeRegion<FMT, 1>(job, res, u, f, x0, y0, zb, cb, lds); break;
+        default: cubeRegion<FMT, 2>(job, res, u, f, x0, y0, zb, cb, lds); break;
     }
 }
 
@@ -966,16 +1131,20 @@ hipError_t renderVplCubes(const float* pos, const uint32_t* colors, int count, i
         const size_t entriesMax = (size_t)batch * 6 * (size_t)stride;
         CubeJob job{pos, colors, count, vpls, updates, first, batch, entries, nearPlane, cull, stride,
                     reinterpret_cast<uint32_t*>(scratch), scratch + entriesMax, scratch + 2 * entriesMax};
-        hipLaunchKernelGGL(clearIntsKernel, dim3((unsigned)((batch * 6 + 255) / 256)), dim3(256), 0, s, job.listCounts,
-                           batch * 6);
-        if (count > 0)
+        const int wc = withDiffuse ? 1 : 0;
+        const bool brief = count <= kShort;
+        if (!brief) {
+            hipLaunchKernelGGL(clearIntsKernel, dim3((unsigned)((batch * 6 + 255) / 256)), dim3(256), 0, s,
+                               job.listCounts, batch * 6);
             hipLaunchKernelGGL(cubeFaceListKernel,
                                dim3((unsigned)((count + kListBlock - 1) / kListBlock), (unsigned)batch),
                                dim3(kListBlock), 0, s, job, res, rpe);
-        const int wc = withDiffuse ? 1 : 0;
+        }
         const long tiles = 4L * batch * 6 * rpe * rpe;
 #define SGI_CUBE_RASTER(F)                                                                                            \
-    if (drawnByBlocks(tiles, count, 0))                                                                               \
+    if (brief)                                                                                                        \
+        hipLaunchKernelGGL(cubeShortKernel<F>, dim3((unsigned)(tiles / 4)), dim3(kShort), 0, s, job, res, rpe, dist, diffuse, wc); \
+    else if (drawnByBlocks(tiles, count, 0))                                                                          \
         hipLaunchKernelGGL((cubeRasterKernel<F, 4>), dim3((unsigned)tiles), dim3(256), 0, s, job, res, rpe, dist, diffuse, wc); \
     else                                                                                                              \
         hipLaunchKernelGGL((cubeRasterKernel<F, 1>), dim3((unsigned)tiles), dim3(64), 0, s, job, res, rpe, dist, diffuse, wc)

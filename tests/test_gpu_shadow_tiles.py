@@ -102,13 +102,15 @@ def _layers(n):
 
 
 # far: every triangle of a wave compares false with a NaN, which nothing is nearer than
-@pytest.mark.parametrize("fmt", [_abi.TEXEL_UNORM16, _abi.TEXEL_F32])
+@pytest.mark.parametrize("n,fmt", [(256, _abi.TEXEL_UNORM16), (256, _abi.TEXEL_F32), (300, _abi.TEXEL_UNORM16),
+                                   (700, _abi.TEXEL_F32)])
 @pytest.mark.parametrize("far,vertex", [(float("nan"), None), (float("inf"), None), (0.0, None), (-30.0, None),
                                         (120.0, float("nan")), (120.0, float("inf")), (120.0, -float("inf"))])
-def test_cubes_not_finite(far, vertex, fmt):
-    """Far planes that bound nothing and vertices that are nowhere, with 256 wide triangles in a tile."""
+def test_cubes_not_finite(far, vertex, n, fmt):
+    """Far planes that bound nothing and vertices that are nowhere, with n wide triangles in a tile: drawn by
+    regions, by a wave a tile and by four."""
     torch = require_gpu()
-    pos, col = _layers(256)
+    pos, col = _layers(n)
     if vertex is not None:
         pos[5, 1, 0] = pos[70, 2] = pos[200, 0, 2] = vertex
     vpls = np.zeros((3, _abi.VPL_FLOATS), np.float32)
@@ -122,7 +124,7 @@ def test_cubes_not_finite(far, vertex, fmt):
     kinds = {_abi.TEXEL_F32: torch.float32, _abi.TEXEL_UNORM16: torch.int16, None: torch.int32}
     z, c, cz, cc = _atlases(3, res, fmt, lambda sh, f: torch.full(sh, 3, dtype=kinds[f], device="cuda"))
     d = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()  # noqa: E731
-    print(f"[tiles] cubes far {far} vertex {vertex} fmt {fmt}", flush=True)
+    print(f"[tiles] cubes far {far} vertex {vertex} triangles {n} fmt {fmt}", flush=True)
     GiPass(64, 64).render_vpl_cubes(d(pos), d(col.view(np.int32)), d(vpls), d(up), d(ent), cz, cc,
                                     cull=_abi.CULLING_NONE)
     torch.cuda.synchronize()
@@ -176,3 +178,45 @@ def test_every_light_of_a_call_in_batches():
     for u in pick:
         assert z[u].tobytes() == hz.reshape(500, 6, 16, 16)[u].tobytes(), f"distance of light {u}"
         assert np.array_equal(c.view(np.uint32)[u], hc.reshape(500, 6, 16, 16)[u]), f"colour of light {u}"
+
+
+# meshes of one to 256 triangles, drawn by regions: 16 and 17 in one (in their order, and near ones first),
+# sides that cut a region and a lane's 2x2 texels
+@pytest.mark.parametrize("n,res,fmt,cull", [
+    (1, 32, _abi.TEXEL_F32, _abi.CULLING_NONE), (16, 31, _abi.TEXEL_F16, _abi.CULLING_NONE),
+    (17, 33, _abi.TEXEL_UNORM16, _abi.CULLING_NONE), (64, 1, _abi.TEXEL_F32, _abi.CULLING_CCW),
+    (65, 47, _abi.TEXEL_F32, _abi.CULLING_CW), (255, 64, _abi.TEXEL_F16, _abi.CULLING_NONE),
+    (256, 47, _abi.TEXEL_UNORM16, _abi.CULLING_NONE), (257, 47, _abi.TEXEL_UNORM16, _abi.CULLING_NONE)])
+@pytest.mark.parametrize("kind", ["layers", "ties", "city"])
+def test_cubes_of_few_triangles(n, res, fmt, cull, kind):
+    """Layers over each other from near to far and back, the same triangle n times and within a step of each
+    format (the first of equal keys stays), and a part of a city: the oracle's bits."""
+    torch = require_gpu()
+    rng = np.random.default_rng(n)
+    s, pos, col = _city(30, 3)
+    vpls = s.vpls()[0][:3].copy()
+    if kind == "city":
+        pos, col = pos[:n], col[:n]
+    else:
+        pos, col = _layers(n)
+        if kind == "ties":
+            pos = np.repeat(pos[:1], n, 0)
+            pos[n // 2:] *= np.float32(1.0) + (rng.integers(-6, 7, (n - n // 2, 1, 1)) * 2.0 ** -18).astype(np.float32)
+        pos = np.ascontiguousarray(pos[rng.permutation(n)])
+        vpls[:, 0:3] = [[0, 0, 0], [0.3, -0.2, 0.1], [-0.5, 0.4, -1.0]]
+        vpls[:, 13] = [100.0, 300.0, 40.0]
+    col = (np.arange(n, dtype=np.uint32) * 0x010307 + 5)  # every triangle its own
+    ent = np.stack([np.zeros(3, np.int32), np.arange(3, dtype=np.int32)], 1)
+    kinds = {_abi.TEXEL_F32: torch.float32, _abi.TEXEL_F16: torch.float16, _abi.TEXEL_UNORM16: torch.int16,
+             None: torch.int32}
+    z, c, cz, cc = _atlases(3, res, fmt, lambda sh, f: torch.full(sh, 3, dtype=kinds[f], device="cuda"))
+    d = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()  # noqa: E731
+    print(f"[tiles] cubes of {n} triangles ({kind}) res {res} fmt {fmt} cull {cull}", flush=True)
+    up = np.arange(3, dtype=np.int32)
+    GiPass(64, 64).render_vpl_cubes(d(pos), d(col.view(np.int32)), d(vpls), d(up), d(ent), cz, cc, cull=cull)
+    torch.cuda.synchronize()
+    hk = {_abi.TEXEL_F32: np.float32, _abi.TEXEL_F16: np.float16, _abi.TEXEL_UNORM16: np.uint16, None: np.uint32}
+    hz, hc, hcz, hcc = _atlases(3, res, fmt, lambda sh, f: np.zeros(sh, hk[f]))
+    orc.render_vpl_cubes(pos, col, vpls, up, ent, _abi.REFERENCE_VPL_NEAR_PLANE, hcz, hcc, cull=cull)
+    assert z.cpu().numpy().tobytes() == hz.tobytes()
+    assert np.array_equal(c.cpu().numpy().view(np.uint32), hc)
