@@ -870,7 +870,10 @@ __global__ __launch_bounds__(kListBlock) void csmListKernel(CsmJob job, int regi
         off += w < wave ? waveCount[w] : 0;
         total += waveCount[w];
     }
-    if (threadIdx.x == 0) base = total ? atomicAdd(job.counts + c, total) : 0;
+    if (threadIdx.x == 0) {
+        if (gridDim.x == 1) job.counts[c] = total;  // the only block: nothing to add to, or to clear before
+        base = gridDim.x > 1 && total ? atomicAdd(job.counts + c, total) : 0;
+    }
     __syncthreads();
     if (keep) {
         const size_t e = (size_t)c * job.stride + base + off + __popcll(bal & ((1ull << lane) - 1ull));
@@ -1103,10 +1106,10 @@ hipError_t renderCsm(const float* pos, int count, int keepSign, float slope, int
     job.tris = scratch + 2 * entries;
     job.counts = (int32_t*)(scratch + 12 * entries);
     const int rpe = (res + kRegion - 1) / kRegion;
-    hipLaunchKernelGGL(clearIntsKernel, dim3(1), dim3(64), 0, s, job.counts, SGI_NUM_CASCADES);
-    if (count > 0)
-        hipLaunchKernelGGL(csmListKernel, dim3((unsigned)((count + kListBlock - 1) / kListBlock), SGI_NUM_CASCADES),
-                           dim3(kListBlock), 0, s, job, rpe);
+    const int listBlocks = max(1, (count + kListBlock - 1) / kListBlock);
+    if (listBlocks > 1)
+        hipLaunchKernelGGL(clearIntsKernel, dim3(1), dim3(64), 0, s, job.counts, SGI_NUM_CASCADES);
+    hipLaunchKernelGGL(csmListKernel, dim3((unsigned)listBlocks, SGI_NUM_CASCADES), dim3(kListBlock), 0, s, job, rpe);
     const long tiles = 4L * SGI_NUM_CASCADES * rpe * rpe;
     if (drawnByBlocks(tiles, count, 4096))
         hipLaunchKernelGGL(csmRasterKernel<4>, dim3((unsigned)tiles), dim3(256), 0, s, job, rpe, depth);
