@@ -45,3 +45,16 @@ def test_taa_history_alignment(shift):
     torch.cuda.synchronize()
     assert np.array_equal(dst.cpu().numpy().view(np.uint32), orc.taa_history(v).view(np.uint32))
     assert bool((buf[1, :shift] == 0).all()) and bool((buf[1, shift + v.size:] == 0).all())
+
+
+@pytest.mark.parametrize("H,W", [(1, 1), (2, 3), (4, 4), (11, 31), (1, 342), (1, 343), (19, 18)])
+def test_taa_history_remainders(H, W):
+    """One to three values after the fours, and none, at and beside a block's 1024."""
+    torch = require_gpu()
+    v = np.random.default_rng(W).uniform(-0.5, 2.0, (H, W, 3)).astype(np.float32)
+    v.reshape(-1)[:3] = [np.nan, np.inf, -np.inf]
+    dst = torch.full((v.size + 4,), -3.0, dtype=torch.float32, device="cuda")
+    GiPass(W, H, 16, 12).taa_history(torch.from_numpy(v).cuda(), dst[:v.size].view(H, W, 3))
+    torch.cuda.synchronize()
+    assert np.array_equal(dst[:v.size].cpu().numpy().view(np.uint32), orc.taa_history(v).view(np.uint32).reshape(-1))
+    assert bool((dst[v.size:] == -3.0).all())
