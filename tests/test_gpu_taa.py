@@ -36,12 +36,12 @@ def test_taa_bit_exact(with_velocity):
         gi.taa(out, d(hist), None, out)
 
 
-def test_taa_clamp_near_ties():
+@pytest.mark.parametrize("H,W", [(256, 768), (640, 768)])  # the two forms of the clamp
+def test_taa_clamp_near_ties(H, W):
     """Histories within a few ulp of the neighbourhood's least and largest values, which lie a few ulp apart
     or are equal: the tone curve rounds, so that neighbours may come out the wrong way round, and the clamp
     has to choose as the curve's values do.  From 1e-6 to where the curve is 1."""
     torch = require_gpu()
-    H, W = 256, 768
     rng = np.random.default_rng(11)
     cur = np.kron(np.exp(rng.uniform(-14, 8, (H // 4, W // 4, 3))), np.ones((4, 4, 1))).astype(np.float32)
     cur[:8, :8], cur[:8, 8:16], cur[:8, 16:24], cur[:8, 24:32] = 0.0, 1e16, 3e7, 1e-30
