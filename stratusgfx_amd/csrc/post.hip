@@ -41,13 +41,14 @@ __device__ __forceinline__ uint32_t tonemapFast(float x, float invGamma, float m
     return tonemapChannel(x, invGamma);
 }
 
+template <bool EXACT>
 __global__ __launch_bounds__(256) void tonemapKernel(const float* __restrict__ lit, long n, float invGamma,
                                                       float margin, uint32_t* __restrict__ out) {
     const long p = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= n) return;
     const float r = lit[3 * p], g = lit[3 * p + 1], b = lit[3 * p + 2];
-    out[p] = tonemapFast(r, invGamma, margin) | (tonemapFast(g, invGamma, margin) << 8) |
-             (tonemapFast(b, invGamma, margin) << 16) | 0xFF000000u;
+    const auto code = [&](float x) { return EXACT ? tonemapChannel(x, invGamma) : tonemapFast(x, invGamma, margin); };
+    out[p] = code(r) | (code(g) << 8) | (code(b) << 16) | 0xFF000000u;
 }
 
 // ---- TAA history (PerformTaaPostFx_'s copy, StratusRendererBackend.cpp:2342-2349)
@@ -389,13 +390,22 @@ hipError_t fxaa(const uint32_t* in, int W, int H, float contrastThreshold, float
     return hipGetLastError();
 }
 
+// Pixels below which every code takes the exact form: with few waves the estimate and, for a lane near a tie,
+// the pow behind it are the longer chain.  A city's frame, us with the estimate / without: 64x64 6.03 / 3.20,
+// 320x180 4.12 / 3.28, 480x270 4.01 / 3.86, 560x315 4.20 / 4.52, 640x360 4.16 / 5.17, 4K 27.2 / 87.7.
+constexpr long kTonemapSmall = 150000;
+
 hipError_t tonemap(const float* lit, long n, float gamma, uint32_t* out, hipStream_t s) {
     if (n <= 0) return hipSuccess;
     const float invGamma = 1.0f / gamma;  // 1.0 / gamma (:113)
-    // 2 always takes the exact form: powers that the estimate's error bound does not hold for
-    const float margin = invGamma > 0.0f && invGamma <= 16.0f ? 2e-4f * (invGamma > 1.0f ? invGamma : 1.0f) : 2.0f;
-    hipLaunchKernelGGL(tonemapKernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, lit, n, invGamma, margin,
-                       out);
+    // the estimate's error bound holds for these powers
+    const bool bounded = invGamma > 0.0f && invGamma <= 16.0f;
+    const dim3 grid((unsigned)((n + 255) / 256));
+    if (bounded && n >= kTonemapSmall)
+        hipLaunchKernelGGL(tonemapKernel<false>, grid, dim3(256), 0, s, lit, n, invGamma,
+                           2e-4f * (invGamma > 1.0f ? invGamma : 1.0f), out);
+    else
+        hipLaunchKernelGGL(tonemapKernel<true>, grid, dim3(256), 0, s, lit, n, invGamma, 0.0f, out);
     return hipGetLastError();
 }
 
