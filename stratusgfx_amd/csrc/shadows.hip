@@ -342,13 +342,13 @@ __device__ __forceinline__ float edgeError(f3 a, f3 b, f3 c) {
     return 0x1p-20f * gmax(dot(a, a), gmax(dot(b, b), dot(c, c)));
 }
 
-// A lower bound of the view depth of the triangle's fragments among rays within h of (midS, midT) on each
-// axis, kFLOAT_MAX where it has none.  A fragment needs e0, e1, e2 all of V's sign (or zero): the view depth
+// Whether the triangle may have a fragment among the rays within h of (midS, midT) on each axis, and a lower
+// bound of their view depth.  A fragment needs e0, e1, e2 all of V's sign (or zero): the view depth
 // V / (e0 + e1 + e2) is positive.  So a rectangle over which one edge, after V's sign, stays below -4 err
 // has no fragment, and where there are some their view depth is at least |V| over the largest sum of the
 // edges.
-__device__ __forceinline__ float nearestDepth(const float4* e, float V, float err, float midS, float midT, float h,
-                                              float farP) {
+__device__ __forceinline__ bool mayCover(const float4* e, float V, float err, float midS, float midT, float h,
+                                         float farP, float& nearest) {
     const float sg = V < 0.0f ? -1.0f : 1.0f;
     float most = 0.0f;
     bool out = false;
@@ -358,8 +358,10 @@ __device__ __forceinline__ float nearestDepth(const float4* e, float V, float er
         out = out || top < -4.0f * err;
         most += top + 4.0f * err;
     }
+    if (out) return false;
     const float t = fabsf(V) * frcp(most) * (1.0f - 0x1p-12f);
-    return out ? kFLOAT_MAX : (most > 1e-30f && t < farP ? t : (most > 1e-30f ? farP : 0.0f));
+    nearest = most > 1e-30f && t < farP ? t : (most > 1e-30f ? farP : 0.0f);
+    return true;
 }
 
 struct CubeLds {
@@ -479,8 +481,7 @@ __device__ __forceinline__ void cubeTile(const CubeJob& job, int res, int u, int
                                  faceAxes<AXIS>(neg, C2, tiny ? 0.0f : V)};
             lds.stage[lane] = StagedTri{e[0], e[1], e[2]};
             const float err = edgeError(a, b, c);
-            nearest = nearestDepth(e, V, err, midS, midT, h, farP);
-            if (nearest != kFLOAT_MAX) {
+            if (mayCover(e, V, err, midS, midT, h, farP, nearest)) {
                 float m[3], s[3], t3[3];
 #pragma unroll
                 for (int i = 0; i < 3; ++i) {
@@ -537,12 +538,11 @@ __device__ __forceinline__ void cubeTile(const CubeJob& job, int res, int u, int
         while (true) {
             const float first = -waveMax(-nearest);
             const float last = waveMax(fmaxf(fmaxf(hi[0], hi[1]), fmaxf(hi[2], hi[3])));
-            if (first > last || first == kFLOAT_MAX) break;
+            // (first NaN: the far plane is, and nothing is nearer.  Otherwise the lane that holds it is taken
+            // below, so the passes end.)
+            if (first > last || !(first < kFLOAT_MAX)) break;
             const bool now = nearest <= fmaxf(4.0f * first, 4.0f * job.nearPlane) && !(nearest > last);
             uint64_t todo = __ballot(now);
-            // No lane may be taken only where every one compares false: a NaN far plane, nearer than which
-            // nothing is.  Without this the pass would repeat for ever.
-            if (todo == 0) break;
             nearest = now ? kFLOAT_MAX : nearest;
             StagedTri next = lds.stage[__builtin_ctzll(todo)];
             while (todo) {
@@ -673,9 +673,8 @@ __device__ __forceinline__ void cubeRegion(const CubeJob& job, int res, int u, i
             const auto edge = [&](int i) { return 2.0f * (float)i / (float)res - 1.0f; };
             const float4 e[3] = {faceAxes<AXIS>(neg, C0, V), faceAxes<AXIS>(neg, cross3(c, a), __int_as_float(k)),
                                  faceAxes<AXIS>(neg, cross3(a, b), 0.0f)};
-            nearest = nearestDepth(e, V, edgeError(a, b, c), edge(x0 + kRegion / 2), edge(y0 + kRegion / 2),
-                                   (float)(kRegion - 1) / (float)res, farP);
-            keep = nearest != kFLOAT_MAX &&
+            keep = mayCover(e, V, edgeError(a, b, c), edge(x0 + kRegion / 2), edge(y0 + kRegion / 2),
+                            (float)(kRegion - 1) / (float)res, farP, nearest) &&
                    !outsideFrustum(m, s, t, edge(x0), edge(min(x0 + kRegion, res)), edge(y0),
                                    edge(min(y0 + kRegion, res)), job.nearPlane, farP);
             tri = StagedTri{e[0], e[1], e[2]};
