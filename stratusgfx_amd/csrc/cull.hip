@@ -243,9 +243,10 @@ __global__ __launch_bounds__(256) void colorVplsKernel(CubeArgs diffuse, CubeArg
 // A tile-culling block's LDS: the per-pixel components that stage 1 sums (six planes at once, three at a
 // time for 32x32 tiles), each plane 4 floats longer than the tile so that the summing lanes read different
 // banks; then, in the same words, stage 2's histogram (256 counters), compacted slot list (kListCap) and
-// ratio codes (a byte per VPL), and over the codes the candidates' keys.  6.5 KB for 8x8 and 16x16 tiles:
-// 24 one-wave blocks per CU.  (Room for 3168 codes in 6.2 KB is 1-5 % faster up to 2048 VPLs, and 4096 then
-// scan twice: 163 us and not 109.)
+// ratio codes (a byte per VPL), and over the codes the candidates' keys.  6.5 KB for 8x8 and 16x16 tiles, with
+// room for every VPL that a frame may hold.  (Its last 288 B are for the codes past 4192: 16x16 tiles of a
+// 1080p frame take 32.4 us instead of 34.1 without them at 512 VPLs, 101.6 and 102.3 at 4096, and, scanning
+// twice, 154 instead of 108 at 4400.)
 constexpr int kListCap = 512, kKeyCap = 256;
 template <int TS>
 struct CullLds {

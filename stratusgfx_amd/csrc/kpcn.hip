@@ -1452,8 +1452,9 @@ __global__ __launch_bounds__(256) void lossKernel(const float* __restrict__ out,
         }
         // Both sums in one request: the atomics on this line, one request at a time, bound the kernel
         // (8100 blocks at 1080p: 223 us with two requests a block, 123 with one). Fewer, larger
-        // blocks would take less, but the rounding of the running FP32 sums, and so the reported
-        // loss, depends on the addends (constant regions give equal ones): 3e-5 on some frames.
+        // blocks would take less, but the running FP32 sums round by their addends (constant
+        // regions give equal ones), and the reported loss with them: 3e-5 on some frames.  (The
+        // blocks' sums added in their order by one block would round as now, without atomics.)
         s1 = __shfl(s1, 0);
         if (t < 2) atomicAdd(&lossSums[t], t == 0 ? s0 : s1);
     }
